@@ -180,3 +180,29 @@ def test_qk_norm_rope_store_qwen3_32b_long_workload(pkg, dev):
                                                 kc0, kc0.copy(), eps=1e-6, rope_theta=1e6)
     _close(u16(q_out[idx]), q_want)
     _close(u16(flat_k[slots[idx]]), kc_want.reshape(sel.size, hkv, d))
+
+
+@pytest.mark.parametrize("h,hkv", [(16, 8), (32, 8), (64, 8), (5, 1)])
+def test_qk_norm_rope_store_few_tokens_bit_identical(pkg, dev, h, hkv):
+    """Launches of few tokens deal a token's rows to several waves: each
+    token's outputs equal, bit for bit, those of a launch of 4 200 tokens
+    (one wave a token), at counts on both sides of every change."""
+    import torch
+    d, bs, t_all = 128, 32, 4200
+    gen = torch.Generator(device=dev).manual_seed(5)
+    rand = lambda *s: torch.randn(s, generator=gen, device=dev).to(torch.bfloat16)  # noqa: E731
+    q, k, v, qw, kw = rand(t_all, h, d), rand(t_all, hkv, d), rand(t_all, hkv, d), rand(d), rand(d)
+    pos = torch.randint(0, 40960, (t_all,), generator=gen, device=dev, dtype=torch.int32)
+    slots = torch.arange(t_all, device=dev, dtype=torch.int32)
+    slots[::7] = -1
+    run = lambda n, pool: pkg.qk_norm_rope_store(q[:n], k[:n], v[:n], qw, kw, pos[:n], slots[:n], pool,  # noqa: E731
+                                                 eps=1e-6, rope_theta=1e6)
+    pool_all = torch.zeros((2, t_all // bs + 1, bs, hkv, d), dtype=torch.bfloat16, device=dev)
+    want, _ = run(t_all, pool_all)
+    for n in (1, 3, 511, 512, 513, 1024, 1025, 2048, 2049, 4096, 4097):
+        pool = torch.zeros_like(pool_all)
+        got, _ = run(n, pool)
+        assert torch.equal(got.view(torch.int16), want[:n].view(torch.int16)), n
+        assert torch.equal(pool.flatten(1, 2)[:, :n].view(torch.int16),
+                           pool_all.flatten(1, 2)[:, :n].view(torch.int16)), n
+        assert not pool.flatten(1, 2)[:, n:].any(), n

@@ -2,10 +2,11 @@
 // projections and attention (vllm/model/qwen3.py:286-299), in one pass over
 // the new tokens.
 //
-// One wavefront per token.  Lane p first evaluates the rotation of pair p
-// (d/2 = 64 pairs) for the token's position; then the wave walks the token's
-// H + 2*Hkv rows four at a time, one row per 16-lane group, each lane owning
-// 8 contiguous elements (4 rotation pairs) of the row:
+// One wavefront per token, or several that share the token's rows when there
+// are few tokens (rope_part_bits).  Lane p first evaluates the rotation of
+// pair p (d/2 = 64 pairs) for the token's position; then the wave walks its
+// share of the token's H + 2*Hkv rows four at a time, one row per 16-lane
+// group, each lane owning 8 contiguous elements (4 rotation pairs) of the row:
 //   q row:  RMSNorm (16-lane sum of squares), scale, RoPE -> q_out
 //   k row:  RMSNorm, scale, RoPE -> k_cache[slot]
 //   v row:  copy -> v_cache[slot]
@@ -48,6 +49,7 @@ struct RopeParams {
   float eps;
   float pos_div;  // linear / dynamic rope scaling factor (positions / factor)
   int32_t scale_pos;
+  int32_t part_bits;  // log2 of the waves a token's rows are dealt to
   uint32_t inv_freq[kRopePairs / 2];  // bf16 pairs: pair 2i in the low half
 };
 
@@ -78,8 +80,13 @@ template <int kRowsInFlight, bool kNtStore>
 __global__ void __launch_bounds__(256)
 qk_norm_rope_store_kernel(RopeParams p) {
   const int lane = threadIdx.x & 63;
-  const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t gw = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t t = gw >> p.part_bits;
   if (t >= p.num_tokens) return;
+  // this wave's share of the token's rows: batch `part` of every `parts`
+  const int part = (int)gw & ((1 << p.part_bits) - 1);
+  const int first = part * 4 * kRowsInFlight;
+  const int step = (4 * kRowsInFlight) << p.part_bits;
   const int i16 = lane & 15;
   const int g = lane >> 4;
   const int nq = p.num_heads;
@@ -97,7 +104,7 @@ qk_norm_rope_store_kernel(RopeParams p) {
   u32x4 x[kRowsInFlight];
 #pragma unroll
   for (int u = 0; u < kRowsInFlight; ++u) {
-    const int r = 4 * u + g;
+    const int r = first + 4 * u + g;
     if (r < rows) x[u] = ld16_stream(row_src(r) + 8 * i16);
   }
 
@@ -128,9 +135,9 @@ qk_norm_rope_store_kernel(RopeParams p) {
     cache_off = pg * p.page_stride + (slot - pg * p.page_size) * p.slot_stride;
   }
 
-  for (int r0 = 0; r0 < rows; r0 += 4 * kRowsInFlight) {
+  for (int r0 = first; r0 < rows; r0 += step) {
     u32x4 nx[kRowsInFlight];
-    const int r1 = r0 + 4 * kRowsInFlight;
+    const int r1 = r0 + step;
     // next batch in flight while this one is computed
 #pragma unroll
     for (int u = 0; u < kRowsInFlight; ++u) {
@@ -177,6 +184,24 @@ qk_norm_rope_store_kernel(RopeParams p) {
 #pragma unroll
     for (int u = 0; u < kRowsInFlight; ++u) x[u] = nx[u];
   }
+}
+
+// log2 of the waves a token's rows are dealt to.  With few tokens the launch
+// is a serial chain, not a stream: one wave walks 32 to 80 rows in batches of
+// 8 or 16, each batch waiting for its loads.  Dealing the batches to 2, 4 or 8
+// waves (each evaluates the rotation again) shortens the chain while the chip
+// still has room for them: up to kRopeWaves waves, and no more parts than
+// there are 8-row batches.  Measured over back-to-back launches, one wave a
+// token -> this rule: 32 / 8 heads 4 tokens 9.0 -> 4.7 us, 256 10.8 -> 4.9,
+// 1000 11.1 -> 8.2, 2000 15.5 -> 13.0; 64 / 8 heads 4 tokens 13.4 -> 5.2,
+// 1000 17.7 -> 11.9.  Past the limit the extra waves only repeat the rotation
+// (16 / 8 heads, 4096 tokens: 16.0 us with one, 17.4 with two, 18.7 with
+// four).
+constexpr int64_t kRopeWaves = 4096;
+static int rope_part_bits(int64_t tokens, int64_t rows) {
+  int bits = 0;
+  while (bits < 3 && (tokens << (bits + 1)) <= kRopeWaves && (8 << bits) < rows) ++bits;
+  return bits;
 }
 
 // bf16 value of x (round to nearest even), as float
@@ -274,7 +299,8 @@ extern "C" int pa_qk_norm_rope_store(const uint16_t* q, int64_t q_tok_stride, in
     }
     prm.inv_freq[i] = w;
   }
-  const int64_t blocks = ((int64_t)num_tokens + 3) / 4;
+  prm.part_bits = rope_part_bits(num_tokens, (int64_t)num_heads + 2 * (int64_t)num_kv_heads);
+  const int64_t blocks = (((int64_t)num_tokens << prm.part_bits) + 3) / 4;
   if (num_heads + 2 * num_kv_heads >= 64)
     qk_norm_rope_store_kernel<4, true><<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(prm);
   else
