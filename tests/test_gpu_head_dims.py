@@ -3,7 +3,9 @@
 pa_prefill, pa_decode and pa_mixed take any head size that is a multiple of 16 from
 16 to 256 (the reference only asks q and the pages to agree,
 prefill_paged_attention.py:199-203, decode_paged_attention.py:356-360);
-sizes other than 128 run the kernels of csrc/any_head.hip.  The cases cover
+sizes other than 128 run the kernels of csrc/any_head.hip, and the prefill at
+64, 96 and 256 over common page sizes the tiled kernel (prefill_heads.hip).
+The cases cover
 the head sizes of common model families (64, 80, 96, 256) and the edges
 (16, 48, 240), head groups from 1 to 40, page sizes that do and do not
 divide 32-token steps, the soft cap, cached prefixes, rows that see no key,
@@ -43,6 +45,59 @@ def test_prefill_head_dims(pkg, dev, lens, h, hkv, bs, d):
     pb = wl.make_prefill(lens, num_heads=h, num_kv_heads=hkv, page_size=bs, head_dim=d,
                          rng=np.random.default_rng(sum(lens) + d))
     _prefill(pkg, dev, pb, seed=d)
+
+
+@pytest.mark.parametrize("d,tile", [(64, 64), (96, 32), (256, 32)])
+@pytest.mark.parametrize("bs", [16, 32, 64, 256])
+@pytest.mark.parametrize("cap", [None, 8.0])
+def test_prefill_head_dims_tiled(pkg, dev, d, tile, bs, cap):
+    """The tiled kernel's page sizes (prefill_heads.hip), capped and not:
+    lengths on both sides of one tile, of the four-stage ring and of the
+    four-iteration loop, groups whose last rows are idle, every sequence
+    against the oracle."""
+    lens = [1, tile - 1, tile, tile + 1, 4 * tile + 1, 5 * tile, 6 * tile - 1, 7 * tile + 2]
+    pb = wl.make_prefill(lens, num_heads=12, num_kv_heads=2, page_size=bs, head_dim=d,
+                         rng=np.random.default_rng(bs + d))
+    _prefill(pkg, dev, pb, seed=d + bs, soft_cap=cap, use_seam=cap is None)
+
+
+@pytest.mark.parametrize("d", [64, 96, 256])
+def test_prefill_head_dims_tiled_equals_generic(pkg, dev, d):
+    """The same tokens over 32-token pages (tiled kernel) and over 24-token
+    pages (generic kernel), cached prefixes, padded rows and q / out views of
+    wider buffers included: both accumulate in f32 and round P and O to bf16
+    (2^-9 relative each), O(1) values, so they differ by at most 2e-2."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(d)
+    h, hkv = 8, 4
+    new, pre = [70, 1, 133, 300], [0, 500, 61, 127]
+    cu = np.concatenate([[0], np.cumsum(new)])
+    cu_k = np.concatenate([[0], np.cumsum(np.add(new, pre))])
+    t = int(cu[-1]) + 5                                    # five rows past the sequences
+    rand = lambda *s: torch.randn(s, generator=gen, device=dev).to(torch.bfloat16)  # noqa: E731
+    q = rand(t, h + 3, d)[:, 1:h + 1]
+    ctx = [rand(2, n, hkv, d) for n in np.diff(cu_k)]
+    i32 = lambda a: torch.as_tensor(np.asarray(a, np.int32), device=dev)  # noqa: E731
+    pos = i32(np.concatenate([np.arange(p, p + n) for n, p in zip(new, pre)] + [np.zeros(5)]))
+    outs = []
+    for bs in (32, 24):
+        pages = [-(-int(n) // bs) for n in np.diff(cu_k)]
+        nb = sum(pages) + 2
+        table = np.full((len(new), max(pages)), -1, np.int32)
+        pool = torch.zeros((2, nb, bs, hkv, d), dtype=torch.bfloat16, device=dev)
+        at = 0
+        for b, n in enumerate(pages):
+            table[b, :n] = np.arange(nb - 1 - at, nb - 1 - at - n, -1)
+            at += n
+            rows = torch.nn.functional.pad(ctx[b], (0, 0, 0, 0, 0, n * bs - ctx[b].shape[1]))
+            pool[:, torch.as_tensor(table[b, :n].astype(np.int64), device=dev)] = rows.view(2, n, bs, hkv, d)
+        out = torch.full((t, 2 * h, d), 7.0, dtype=torch.bfloat16, device=dev)[:, h:]
+        got = pkg.prefill_paged_attention(q, pool[0].permute(2, 0, 1, 3), pool[1].permute(2, 0, 1, 3), i32(table),
+                                          i32(cu), pos, pos, max_seqlen_bucket=256, cu_seqlens_k=i32(cu_k), out=out)
+        assert not got[int(cu[-1]):].any() and not got[int(cu[-2]) + 256:int(cu[-1])].any()
+        outs.append(got.float())
+    assert float((outs[0] - outs[1]).abs().max()) <= TOL
+    assert float(outs[0].abs().max()) > 0.5
 
 
 def test_prefill_head_dim_soft_cap_kernel_entry(pkg, dev):

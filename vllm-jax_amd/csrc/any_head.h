@@ -13,6 +13,12 @@ struct DecodeParams;
 // multiples of 16 from 16 to 256 other than 128 (the tuned kernels' size).
 bool any_head_dim(int head_dim);
 
+// Prefill of `p` with the tiled ping-pong kernel at the head sizes and page
+// sizes it is built for (prefill_heads.hip), rows no item covers zeroed;
+// kPrefillNotTiled, with nothing launched, for any other.  Else a PA_* code.
+constexpr int kPrefillNotTiled = 1;
+int prefill_tiled_launch(const char* name, const PrefillParams& p, int head_dim, hipStream_t s);
+
 // Zero pass and prefill of `p` (filled as for the tuned kernel; the work
 // list and pools are not used) with `head_dim`-wide rows.  Returns a PA_*
 // code.

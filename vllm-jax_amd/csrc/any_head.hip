@@ -832,6 +832,10 @@ int prefill_any_launch(const char* name, const PrefillParams& prm, int head_dim,
   if (p.group > 32 * waves)
     return fail(PA_ERR_UNSUPPORTED, "%s: %d q heads per kv head not supported at head_dim %d (max %d)", name,
                 p.group, head_dim, 32 * waves);
+#ifndef PA_PREFILL_PHASES
+  const int tiled = prefill_tiled_launch(name, prm, head_dim, s);
+  if (tiled != kPrefillNotTiled) return tiled;
+#endif
   p.plan = nullptr;
   p.pool = nullptr;
   p.tile_tokens = 32 * waves / p.group;

@@ -8,56 +8,6 @@
 
 namespace pa {
 
-// Output rows the prefill items do not write, for 64 tokens t0 .. t0 + 63
-// (one wave): rows outside all sequences (before cu_q[0], from cu_q[batch]
-// on) and rows at offset >= max_seqlen_q inside their sequence (the
-// reference drops those too: its scatter only covers the first
-// max_seqlen_bucket rows, prefill...:384-388) are zeroed.  A lane checks one
-// token; the wave zeroes the rows it found, one after the other.
-__device__ void prefill_zero_rows(const PrefillParams& p, int64_t t0) {
-  const int lane = threadIdx.x & 63;
-  const int64_t t = t0 + lane;
-  const int32_t* cu_q = p.cu_q;
-  const int batch = p.batch;
-  bool zero = t < p.num_tokens;
-  if (zero && batch > 0 && t >= cu_q[0] && t < cu_q[batch]) {
-    // last b with cu_q[b] <= t
-    int lo = 0, hi = batch;  // invariant: cu_q[lo] <= t < cu_q[hi]
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (cu_q[mid] <= t) lo = mid;
-      else hi = mid;
-    }
-    zero = t - cu_q[lo] >= p.max_seqlen_q;
-  }
-  uint64_t todo = __ballot(zero);
-  const int chunks = p.num_heads * (kPHeadDim / 8);
-  while (todo) {
-    const int k = __ffsll((unsigned long long)todo) - 1;
-    todo &= todo - 1;
-    uint16_t* row = p.out + (t0 + k) * p.o_ts;
-    for (int c = lane; c < chunks; c += 64) {
-      const int hh = c / (kPHeadDim / 8);
-      st16(row + hh * p.o_hs + (c - hh * (kPHeadDim / 8)) * 8, u32x4{0, 0, 0, 0});
-    }
-  }
-}
-
-// kZero (launches without a work list): workgroups past the items zero the
-// rows no item writes, 512 tokens each, in place of a launch of their own.
-template <bool kSoftCap, int kPaging, bool kZero = false>
-__global__ void __launch_bounds__(kThreads, 1)
-prefill_kernel(PrefillParams p) {
-  if constexpr (kZero) {
-    const int64_t items = (int64_t)p.n_qtiles * p.batch * p.num_kv_heads;
-    if (blockIdx.x >= items) {  // uniform over the workgroup
-      prefill_zero_rows(p, ((int64_t)blockIdx.x - items) * kThreads + 64 * (threadIdx.x >> 6));
-      return;
-    }
-  }
-  prefill_body<kSoftCap, kPaging>(p, blockIdx.x);
-}
-
 // The item of workgroup `bid` with the pools: every XCD walks the whole list
 // (n items, one kv head of every entry, as prefill_resolve deals them), but
 // only its first n - s items statically (workgroup 8 k + x runs XCD x's k-th

@@ -6,6 +6,9 @@
 // the MFMA dimension makes every K/V tile staged in LDS serve G x tokens rows.
 // One workgroup per CU, two waves per SIMD.
 //
+// Head size 128 (prefill.hip, mixed.hip) and, over the common page sizes, 64,
+// 96 and 256 (prefill_heads.hip); tile sizes below are those of 128.
+//
 // KV tiles of 64 tokens go through a 4-stage LDS ring filled by direct
 // global->LDS loads (global_load_lds_dwordx4) through the block table, issued
 // two to three tiles ahead of use.  Per tile and wave:
@@ -87,10 +90,10 @@ struct PrefillParams {
 };
 
 // How the tile loads find their pages.  kPageLane: each lane looks up its
-// row's page (any page size).  kPageTile: pages of a multiple of 64 tokens
-// hold whole tiles, one scalar page base per tile.  kPageWave: pages of 16 or
-// 32 tokens; a wave's 8 rows of a tile lie in one page, one scalar page base
-// per wave and tile.
+// row's page (any page size).  kPageTile: pages of a multiple of the tile's
+// tokens hold whole tiles, one scalar page base per tile.  kPageWave: pages of
+// 16 or 32 tokens; a wave's rows of a tile (at most 8) lie in one page, one
+// scalar page base per wave and tile.
 constexpr int kPageLane = 0, kPageTile = 1, kPageWave = 2;
 
 // One entry of the work list: a (sequence, q tile) pair with the sequence's
@@ -114,10 +117,52 @@ __device__ __forceinline__ u32x4 ds_read16(lds_cbytes a) {
   return *reinterpret_cast<const u32x4 __attribute__((address_space(3)))*>(a);
 }
 
-// Physical 16-byte chunk of logical chunk c in tile row r.
-__device__ __forceinline__ int swz(int r, int c) {
-  return c ^ (((r & 3) << 2) | ((r >> 2) & 3));
-}
+// Tile geometry of a head size.  LDS rows are 128, 256 or 512 bytes (the head
+// size rounded up) and a K (or V) tile fills one ring stage of 16 KiB (64
+// tokens at 128, 32 at 256: 32 MFMAs a segment of the loop either way).  Where
+// 128 registers hold a wave's state (64, and 96 without the soft cap) stages
+// are 8 KiB and two workgroups share a CU, so that one's first loads and last
+// stores run under the other's loop: at 64 16 sequences of 1000 to 3000 tokens
+// took 399 us with one workgroup and 128-token tiles, 351 us so.
+template <int D, bool kSoftCap>
+struct PrefillDims {
+  static_assert(D % 16 == 0 && D > 32 && D <= 256, "head size");
+  static constexpr int kRowB = D <= 64 ? 128 : (D <= 128 ? 256 : 512);  // bytes per LDS row
+  static constexpr int kWgs = D <= 64 || (D <= 96 && !kSoftCap) ? 2 : 1;  // workgroups per CU
+  static constexpr int kStageB = 2 * kTileElems / kWgs;  // bytes of a K or V stage
+  static constexpr int kN = kStageB / kRowB;         // kv tokens per tile
+  static constexpr int kBlk = kStageB / 1024 / kWaves;  // 1 KiB blocks of K (and of V) a wave loads per tile
+  static constexpr int kRowChunks = kRowB / 16;      // 16-byte chunks per LDS row
+  static constexpr int kChunks = D / 8;              // of which hold the head's elements
+  static constexpr int kBlkRows = 1024 / kRowB;      // rows of a 1 KiB block (one DMA of a wave)
+  static constexpr int kWaveRows = kBlk * kBlkRows;  // tile rows a wave loads
+  // stages whose blocks of one wave hold its 32 Q (or O) rows
+  static constexpr int kRowStages = 32 * kRowB / (2048 * kBlk);
+  static_assert(kRowStages <= kStages, "a wave's rows fit its own blocks");
+  static constexpr int kKs = D / 16;                 // k-steps of S^T = K Q^T
+  static constexpr int kDt = (D + 31) / 32;          // 32-row blocks of O^T
+  static constexpr int kMt = kN / 32;                // 32-token blocks of S^T
+  static constexpr int kU = kN / 16;                 // 16-token k-steps of O^T += V^T P^T
+  // The QK accumulators start from -m_ref where the registers allow it (16
+  // of them); elsewhere the reference is subtracted from S.
+  static constexpr bool kFoldRef = kRowB == 256 && kWgs == 1;
+  // MFMAs between an LDS read and the MFMA it feeds (at 512-byte rows one
+  // operand's registers fewer: four spilled an address in the loop)
+  static constexpr int kAhead = kRowB < 512 ? kAheadMfma : 3;
+  // Chunk swizzle of tile row r (XORed into the chunk index, low 4 bits of
+  // r): 16 rows' reads of one chunk and a transposing read's 4 rows x 64
+  // bytes both land on distinct banks.
+  static __host__ __device__ constexpr int swz(int r) {
+    return kRowB == 128 ? (((r >> 1) & 1) << 2) | ((r >> 2) & 3) : ((r & 3) << 2) | ((r >> 2) & 3);
+  }
+  // The same for the staged Q and O rows (no transposing reads).
+  static __host__ __device__ constexpr int qswz(int r) { return kRowB == 128 ? (r >> 1) & 7 : r & 15; }
+  // Chunks past the head's elements load a chunk of their own row again: Q
+  // is multiplied by its k-steps only, and O^T rows past D are never stored.
+  static __host__ __device__ constexpr int real_chunk(int c) {
+    return kChunks == kRowChunks || c < kChunks ? c : c - (kRowChunks - kChunks);
+  }
+};
 
 // Work item of workgroup `bid`: (q tile, sequence b, kv head).  Items are
 // ordered from the last q tile down (longest causal rows first).  Within one
@@ -178,6 +223,17 @@ static __shared__ __attribute__((aligned(1024))) uint16_t k_lds[kStages][kTileEl
 static __shared__ __attribute__((aligned(1024))) uint16_t v_lds[kStages][kTileElems];
 static __shared__ int red_max[kWaves], red_min[kWaves];
 
+// LDS byte address of the K (kV = 0) or V (1) ring of kStages stages.
+template <int kStageB, int kV>
+__device__ __forceinline__ uint32_t prefill_ring() {
+  if constexpr (kStageB == 2 * kTileElems) {
+    return (uint32_t)(uintptr_t)(lds_void_ptr)(kV ? &v_lds[0][0] : &k_lds[0][0]);
+  } else {
+    static __shared__ __attribute__((aligned(1024))) uint16_t ring[kStages * kStageB / 2];
+    return (uint32_t)(uintptr_t)(lds_void_ptr)&ring[0];
+  }
+}
+
 // Per-workgroup phase timestamps, only in a build with PA_PREFILL_PHASES
 // (libpaged_attention_phases.so; the library proper has none): s_memrealtime
 // (100 MHz) at the item's start, once its kv range is known, once its first
@@ -215,8 +271,8 @@ __device__ __forceinline__ void prefill_phases_store(unsigned long long t0, unsi
 // a scalar page base: tile row r (< 64) plus a 16-byte chunk (< 128 elements)
 // is r * slot_stride + 8 * chunk elements, 2x that in bytes.  True when that
 // fits int32 for every row (so the byte offset fits uint32 as well).
-inline bool prefill_offsets_fit(int64_t slot_stride) {
-  return slot_stride >= 0 && (kTileN - 1) * slot_stride + kPHeadDim - 1 <= (int64_t)0x7fffffff;
+inline bool prefill_offsets_fit(int64_t slot_stride, int tile_n = kTileN, int head_dim = kPHeadDim) {
+  return slot_stride >= 0 && (tile_n - 1) * slot_stride + head_dim - 1 <= (int64_t)0x7fffffff;
 }
 
 // Row range and kv geometry of prefill sequence b, as prefill_resolve
@@ -302,12 +358,15 @@ __device__ __forceinline__ bool prefill_resolve(const PrefillParams& p, int bid,
 }
 
 // One prefill work item, run by a whole 512-thread workgroup.
-template <bool kSoftCap, int kPaging>
+template <bool kSoftCap, int kPaging, int D = kPHeadDim>
 __device__ __forceinline__ void prefill_run(const PrefillParams& p, const PrefillWork& w) {
+  using A = PrefillDims<D, kSoftCap>;
+  constexpr int kN = A::kN;
   constexpr bool kAligned = kPaging != kPageLane;  // scalar page bases
   PA_PHASE(ph0);
-  auto k_stage = [&](auto c) __attribute__((always_inline)) -> uint16_t* { return k_lds[decltype(c)::value]; };
-  auto v_stage = [&](auto c) __attribute__((always_inline)) -> uint16_t* { return v_lds[decltype(c)::value]; };
+  // LDS byte addresses of the two rings
+  const uint32_t k_lds0 = prefill_ring<A::kStageB, 0>();
+  const uint32_t v_lds0 = prefill_ring<A::kStageB, 1>();
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -330,45 +389,46 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   // rows grow with the token: a wave whose first row has no token has none
   const bool wave_live = 32 * wave < p.tile_tokens * p.group && tok0 + (32 * wave) / p.group < lq_rows;
 
-  // Wave w stages its Q rows and, at the end, its O rows in its own LDS:
-  // 1 KiB blocks 2w and 2w+1 of K and of V in every stage, the only blocks
-  // its own tile loads write (so no other wave's loads or reads can touch
-  // them at those times).  Piece j of stage pair st holds rows 8j .. 8j+7 of
-  // the wave, 256 bytes per row, with 16-byte chunk c of row r stored at
-  // chunk c ^ (r & 15) (conflict-free reads of one chunk from 16 rows).
+  // Wave w stages its Q rows and, at the end, its O rows in its own LDS: its
+  // kBlk 1 KiB blocks of K and of V in every stage, the only blocks its own
+  // tile loads write (so no other wave's loads or reads can touch them at
+  // those times).  Piece j from stage st on holds kWaveRows rows of
+  // the wave, kRowB bytes per row, with 16-byte chunk c of row r stored at
+  // chunk c ^ qswz(r) (conflict-free reads of one chunk from 16 rows).
   auto piece = [&](int st, int j) __attribute__((always_inline)) -> uint32_t {
-    return (uint32_t)(uintptr_t)(lds_void_ptr)((j & 1) ? &v_lds[st + (j >> 1)][0] : &k_lds[st + (j >> 1)][0]) +
-           (uint32_t)(2048 * wave);
+    return ((j & 1) ? v_lds0 : k_lds0) + (uint32_t)((st + (j >> 1)) * A::kStageB + 1024 * A::kBlk * wave);
   };
   // row / group for rows < 256 as (row * gm) >> 24 (exact for group <= 256)
   const uint32_t gm = (0x1000000u + (uint32_t)p.group - 1u) / (uint32_t)p.group;
 
-  // Q tile rows into stages 2 and 3 (free until tile 2 is issued, after the
-  // barrier below), four whole 256-byte rows per load: full cache lines, where
-  // a lane-per-row load would touch 32 lines a quarter each.  Issued before
-  // the position reduction below so that their latencies overlap.
-  bf16x8 qt_op[8];
+  // Q tile rows into the last two stages (or all four), free until the tile
+  // loads are issued after the barrier below, 1 KiB of whole rows per
+  // load: full cache lines, where a lane-per-row load would touch 32 lines a
+  // quarter each.  Issued before the position reduction below so that their
+  // latencies overlap.
+  constexpr int kQSt = kStages - A::kRowStages;
+  bf16x8 qt_op[A::kKs];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = 4 * i + (lane >> 4);
+  for (int i = 0; i < 32 / A::kBlkRows; ++i) {
+    const int r = A::kBlkRows * i + lane / A::kRowChunks;
     const int rw = wave * 32 + r;
     const int tk = (int)(((uint32_t)rw * gm) >> 24);
     const int hd = rw - tk * p.group;
     const int lt = min(tok0 + tk, lq_rows - 1);
-    const int c = (lane & 15) ^ (r & 15);
+    const int c = A::real_chunk((lane & (A::kRowChunks - 1)) ^ A::qswz(r));
     dma16(p.q + (int64_t)(q0 + lt) * p.q_ts + (int64_t)(kvh * p.group + hd) * p.q_hs + 8 * c,
-          piece(2, i >> 1) + 1024 * (i & 1));
+          piece(kQSt, i / A::kBlk) + 1024 * (i % A::kBlk));
   }
   const int qpos = row_ok ? qpos_ld : 0;
   // raw page ids of the first three kv tiles, read while the loads above fly
   int32_t raw_pre[3] = {0, 0, 0};
   // (kPageWave) log2 of the page size, and the table entry of this wave's
-  // rows of tile T: rows 8w .. 8w + 7, or the tile's last row inside the kv
+  // rows of tile T: rows kWaveRows w on, or the tile's last row inside the kv
   // length when they lie past it (a wave's rows never straddle a page)
   const int pg_sh = kPaging == kPageWave ? (p.page_size == 16 ? 4 : 5) : 0;
   auto wave_entry = [&](int T) __attribute__((always_inline)) {
-    const int last = min(max(lk - 1 - T * kTileN, 0), kTileN - 1);
-    return (T * kTileN + min(8 * wave, last)) >> pg_sh;
+    const int last = min(max(lk - 1 - T * kN, 0), kN - 1);
+    return (T * kN + min(A::kWaveRows * wave, last)) >> pg_sh;
   };
   if constexpr (kAligned) {
     if (p.pages_per_seq > 0) {
@@ -376,7 +436,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
           (const __attribute__((address_space(4))) int32_t*)(p.block_tables + (int64_t)b * p.bt_stride);
 #pragma unroll
       for (int i = 0; i < 3; ++i)
-        raw_pre[i] = c[min(kPaging == kPageWave ? wave_entry(i) : i * kTileN / p.page_size, p.pages_per_seq - 1)];
+        raw_pre[i] = c[min(kPaging == kPageWave ? wave_entry(i) : i * kN / p.page_size, p.pages_per_seq - 1)];
     }
   }
 
@@ -400,9 +460,10 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   // Q^T operand (B of S^T): lane (n, h)'s k-step ks is row n, d = 16ks + 8h
   // .. +8, i.e. chunk 2ks + h
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks)
-    qt_op[ks] = as_bf16x8(
-        ds_read16((lds_cbytes)(uintptr_t)(piece(2, n >> 3) + 256 * (n & 7) + 16 * ((2 * ks + h) ^ (n & 15)))));
+  for (int ks = 0; ks < A::kKs; ++ks)
+    qt_op[ks] = as_bf16x8(ds_read16((lds_cbytes)(uintptr_t)(piece(kQSt, n / A::kWaveRows) +
+                                                            A::kRowB * (n & (A::kWaveRows - 1)) +
+                                                            16 * ((2 * ks + h) ^ A::qswz(n)))));
   // read before any wave passes the barrier below (then tile 2 may overwrite
   // stage 2)
   wait_vm_lgkm0<0>();
@@ -410,7 +471,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
     // Q^T scaled by scale * log2 e (rounded to bf16), so that S = K Q^T is in
     // log2 units
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
+    for (int ks = 0; ks < A::kKs; ++ks) {
       const u32x4 w = __builtin_bit_cast(u32x4, qt_op[ks]);
       u32x4 o;
 #pragma unroll
@@ -428,33 +489,34 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   // kv index j is visible to some row iff j < lk and j + kv_pos_off <= qpos_max
   const int64_t kv_hi64 = min((int64_t)lk, (int64_t)qpos_max - kv_pos_off + 1);
   const int kv_hi = kv_hi64 < 0 ? 0 : (int)kv_hi64;
-  const int n_tiles = (kv_hi + kTileN - 1) / kTileN;
+  const int n_tiles = (kv_hi + kN - 1) / kN;
   PA_PHASE(ph1);
   // tiles [0, n_free) need no mask: every token is < lk and visible to every row
   const int64_t free_hi = min((int64_t)lk, (int64_t)qpos_min - kv_pos_off + 1);
-  const int n_free = free_hi < 0 ? 0 : (int)(free_hi / kTileN);
+  const int n_free = free_hi < 0 ? 0 : (int)(free_hi / kN);
 
-  // ---- direct global->LDS tile loader.  A tile is 16 blocks of 1 KiB
-  // (4 rows each); wave w fills blocks kBlk*w .. kBlk*w + kBlk-1 of K and V.
-  // Lane l writes LDS bytes 16*l of a block, i.e. row 4blk + l/16, physical
-  // chunk l%16, so it loads the logical chunk swz(row, l%16) of that token.
-  constexpr int kBlk = 16 / kWaves;
+  // ---- direct global->LDS tile loader.  A tile is kWaves * kBlk blocks of
+  // 1 KiB (kBlkRows rows each); wave w fills blocks kBlk*w .. kBlk*w + kBlk-1 of K
+  // and V.  Lane l writes LDS bytes 16*l of a block, i.e. row kBlkRows blk +
+  // l / kRowChunks, physical chunk l % kRowChunks, so it loads the logical
+  // chunk (physical ^ swz(row)) of that token.
+  constexpr int kBlk = A::kBlk;
   const int32_t* bt_row = p.block_tables + (int64_t)b * p.bt_stride;
-  const int ld_r = lane >> 4;            // row within a 1 KiB block
-  const int ld_p = lane & 15;            // physical chunk
+  const int ld_r = lane / A::kRowChunks;        // row within a 1 KiB block
+  const int ld_p = lane & (A::kRowChunks - 1);  // physical chunk
   const int64_t head_off = (int64_t)kvh * p.head_stride;
   // per-lane element offset of the row within a page; the host guarantees
-  // 63 * slot_stride + 127 <= INT32_MAX (prefill_offsets_fit), so neither
+  // (kN - 1) * slot_stride + D - 1 <= INT32_MAX (prefill_offsets_fit), so neither
   // this nor the byte offset 2 * ld_off below wraps
   uint32_t ld_off[kBlk];
   uint32_t ld_sw[kBlk];  // its swizzled chunk part alone
-  static_assert(kPaging != kPageWave || kBlk == 2, "a wave's rows of a tile must lie in one 16-token page");
+  static_assert(kPaging != kPageWave || A::kWaveRows <= 8, "a wave's rows of a tile must lie in one 16-token page");
   // (kPageWave) tile rows are rows of the wave's page: r mod page size
-  const int row_mask = kPaging == kPageWave ? p.page_size - 1 : kTileN - 1;
+  const int row_mask = kPaging == kPageWave ? p.page_size - 1 : kN - 1;
 #pragma unroll
   for (int i = 0; i < kBlk; ++i) {
-    const int r = 4 * (kBlk * wave + i) + ld_r;
-    ld_sw[i] = (uint32_t)(8 * swz(r, ld_p));
+    const int r = A::kBlkRows * (kBlk * wave + i) + ld_r;
+    ld_sw[i] = (uint32_t)(8 * A::real_chunk(ld_p ^ A::swz(r)));
     ld_off[i] = (uint32_t)((kPaging == kPageWave ? r & row_mask : r) * (int32_t)p.slot_stride) + ld_sw[i];
   }
   // Tile DMA in two steps: tile_addrs() computes this wave's 2*kBlk global
@@ -467,11 +529,11 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
     uint32_t vo[kBlk];      // (aligned) this lane's byte offsets from them
     const uint16_t* g[2 * kBlk];  // (unaligned) this lane's pointers
   };
-  // Aligned pages hold tpp whole tiles: tile j0 = 64 (tpp lp + r) is tile r
+  // Aligned pages hold tpp whole tiles: tile j0 = kN (tpp lp + r) is tile r
   // of table entry lp.  The loop walks (lp, r) incrementally, so no division
   // sits on the softmax wave's path.
-  const int tpp = kPaging == kPageTile ? p.page_size / kTileN : 1;
-  const int64_t tile_stride = (int64_t)kTileN * p.slot_stride;
+  const int tpp = kPaging == kPageTile ? p.page_size / kN : 1;
+  const int64_t tile_stride = (int64_t)kN * p.slot_stride;
   auto page_raw_at = [&](int lp) __attribute__((always_inline)) {
     const __attribute__((address_space(4))) int32_t* c = (const __attribute__((address_space(4))) int32_t*)bt_row;
     // stays inside the table row (only called with n_tiles > 0, so the row
@@ -494,42 +556,40 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
       // never stale); a tile wholly past it reads its row 0.  Selects, no
       // branch.
       const int last = __builtin_amdgcn_readfirstlane(max(lk - 1 - j0, 0));
-      const int last_row = kPaging == kPageWave ? min(last, kTileN - 1) & row_mask : min(last, kTileN - 1);
+      const int last_row = kPaging == kPageWave ? min(last, kN - 1) & row_mask : min(last, kN - 1);
       const uint32_t last_off = (uint32_t)(last_row * (int32_t)p.slot_stride);
 #pragma unroll
       for (int i = 0; i < kBlk; ++i) {
-        const int r = 4 * (kBlk * wave + i) + ld_r;
+        const int r = A::kBlkRows * (kBlk * wave + i) + ld_r;
         a.vo[i] = 2u * (r <= last ? ld_off[i] : last_off + ld_sw[i]);
       }
     } else {
       int32_t pages[kBlk];
 #pragma unroll
       for (int i = 0; i < kBlk; ++i) {
-        const int r = 4 * (kBlk * wave + i) + ld_r;
+        const int r = A::kBlkRows * (kBlk * wave + i) + ld_r;
         const int j = min(j0 + r, lk - 1);
         pages[i] = safe_page(bt_row, j / p.page_size, p.num_pages);
       }
 #pragma unroll
       for (int i = 0; i < kBlk; ++i) {
-        const int r = 4 * (kBlk * wave + i) + ld_r;
+        const int r = A::kBlkRows * (kBlk * wave + i) + ld_r;
         const int j = min(j0 + r, lk - 1);
         const int64_t o = (int64_t)pages[i] * p.page_stride + (int64_t)(j % p.page_size) * p.slot_stride +
-                          head_off + 8 * swz(r, ld_p);
+                          head_off + 8 * A::real_chunk(ld_p ^ A::swz(r));
         a.g[2 * i] = p.k_cache + o;
         a.g[2 * i + 1] = p.v_cache + o;
       }
     }
     return a;
   };
-  const uint32_t k_lds0 = (uint32_t)(uintptr_t)(lds_void_ptr)(&k_lds[0][0]);
-  const uint32_t v_lds0 = (uint32_t)(uintptr_t)(lds_void_ptr)(&v_lds[0][0]);
   auto dma_issue = [&](const TileAddrs& a, int i, int stage) __attribute__((always_inline)) {
-    const uint32_t lds = ((i & 1) ? v_lds0 : k_lds0) + (uint32_t)(stage * kTileElems * 2 + (kBlk * wave + (i >> 1)) * 1024);
+    const uint32_t lds = ((i & 1) ? v_lds0 : k_lds0) + (uint32_t)(stage * A::kStageB + (kBlk * wave + (i >> 1)) * 1024);
     if constexpr (kAligned) dma16s(a.vo[i >> 1], (i & 1) ? a.vb : a.kb, lds);
     else dma16(a.g[i], lds);
   };
   auto issue_tile_raw = [&](int j0, int32_t raw, int stage) __attribute__((always_inline)) {
-    const TileAddrs a = tile_addrs(j0, raw, (j0 / kTileN) % tpp);
+    const TileAddrs a = tile_addrs(j0, raw, (j0 / kN) % tpp);
 #pragma unroll
     for (int i = 0; i < 2 * kBlk; ++i) dma_issue(a, i, stage);
   };
@@ -538,10 +598,12 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   // ---- per-lane LDS read offsets (bytes), fixed for the whole kernel.
   // K (A of S^T): row 32mt + n, logical chunk 2ks + h; the swizzle of a row
   // only depends on its low 4 bits, i.e. on n.
-  const int fn = ((n & 3) << 2) | ((n >> 2) & 3);
-  uint32_t koff[8];
+  // Past 16 chunks the swizzle leaves the chunk's bit 4 alone: +256 bytes.
+  constexpr int kKOff = A::kKs < 8 ? A::kKs : 8, kVOff = A::kDt < 4 ? A::kDt : 4;
+  const int fn = A::swz(n);
+  uint32_t koff[kKOff];
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks) koff[ks] = n * 256 + 16 * ((2 * ks + h) ^ fn);
+  for (int ks = 0; ks < kKOff; ++ks) koff[ks] = k_lds0 + n * A::kRowB + 16 * ((2 * ks + h) ^ fn);
   // V^T (tr16): lane = 16*gamma + s reads row tokbase + 4h + s/4 (+8) and
   // logical column 32dt + 16(gamma%2) + 4(s%4): chunk 4dt + 2(gamma%2) +
   // (s%4)/2, byte 8*(s%2) inside it.  tokbase is a multiple of 16, so the
@@ -549,31 +611,39 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   const int tr_s = lane & 15;
   const int tr_gamma = lane >> 4;
   const int tr_row = 4 * h + (tr_s >> 2);
-  const int f0 = ((tr_row & 3) << 2) | ((tr_row >> 2) & 3);
-  const int f1 = (((tr_row + 8) & 3) << 2) | (((tr_row + 8) >> 2) & 3);
-  uint32_t voff0[4], voff1[4];
+  const int f0 = A::swz(tr_row);
+  const int f1 = A::swz(tr_row + 8);
+  // row + 8 flips bit 1 of the swizzle, so voff1 = (voff0 ^ 32) + 8 rows; at
+  // 512-byte rows it is made from voff0 in every PV (four registers fewer)
+  constexpr bool kV1 = A::kRowB < 512;
+  uint32_t voff0[kVOff], voff1[kVOff];
 #pragma unroll
-  for (int dt = 0; dt < 4; ++dt) {
+  for (int dt = 0; dt < kVOff; ++dt) {
     const int c = 4 * dt + 2 * (tr_gamma & 1) + ((tr_s & 3) >> 1);
-    voff0[dt] = v_lds0 + tr_row * 256 + 16 * (c ^ f0) + 8 * (tr_s & 1);
-    voff1[dt] = v_lds0 + (tr_row + 8) * 256 + 16 * (c ^ f1) + 8 * (tr_s & 1);
+    voff0[dt] = v_lds0 + tr_row * A::kRowB + 16 * (c ^ f0) + 8 * (tr_s & 1);
+    voff1[dt] = v_lds0 + (tr_row + 8) * A::kRowB + 16 * (c ^ f1) + 8 * (tr_s & 1);
   }
 #pragma unroll
-  for (int dt = 0; dt < 4; ++dt) asm volatile("" : "+v"(voff0[dt]), "+v"(voff1[dt]));
+  for (int dt = 0; dt < kVOff; ++dt) {
+    asm volatile("" : "+v"(voff0[dt]));
+    if constexpr (kV1) asm volatile("" : "+v"(voff1[dt]));
+  }
 
-  f32x16 acc_o[4];
+  f32x16 acc_o[A::kDt];
 #pragma unroll
-  for (int dt = 0; dt < 4; ++dt)
+  for (int dt = 0; dt < A::kDt; ++dt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc_o[dt][i] = 0.f;
   float m_ref = 0.f;  // reference max (log2 units) of the accumulators
-  f32x16 neg_mref = {};  // -m_ref in every element: the QK accumulators start from it
-  // running row sums, one per quarter of a tile (four short add chains), of
-  // the f32 exponentials: v_dot2c on the packed P would wait for the matrix
+  constexpr bool kFold = !kSoftCap && A::kFoldRef;
+  f32x16 neg_mref = {};  // (kFold) -m_ref in every element: the QK accumulators start from it
+  // running row sums (up to four short add chains, one per 16-token k-step
+  // of a 64-token tile), of the f32 exponentials: v_dot2c on the packed P would wait for the matrix
   // core, which the other wave of the SIMD keeps busy
-  float l_part[4] = {0.f, 0.f, 0.f, 0.f};
-  f32x16 s_acc[2];  // S^T of the tile between its QK and its softmax
-  bf16x8 pt[4];     // P^T of the tile between its softmax and its PV
+  constexpr int kL = A::kU < 4 ? A::kU : 4;
+  float l_part[kL] = {};
+  f32x16 s_acc[A::kMt];  // S^T of the tile between its QK and its softmax
+  bf16x8 pt[A::kU];      // P^T of the tile between its softmax and its PV
 
   // ---- work pieces.  M(t) = PV(t-1) + QK(t) is MFMA work, SM(t) = softmax of
   // tile t is VALU work.  Waves 0-3 (group A) and 4-7 (group B) share the
@@ -583,26 +653,33 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   // with a workgroup barrier after every segment, so on every SIMD one wave
   // feeds the matrix core while the other one does its softmax (ping-pong).
   auto qk = [&](auto kst) __attribute__((always_inline)) {
-    const lds_cbytes kt = (lds_cbytes)(k_stage(kst));
+    constexpr uint32_t kb = decltype(kst)::value * A::kStageB;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
+    for (int ks = 0; ks < A::kKs; ++ks) {
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        const bf16x8 a = as_bf16x8(ds_read16(kt + koff[ks] + mt * 8192));
+      for (int mt = 0; mt < A::kMt; ++mt) {
+        const bf16x8 a = as_bf16x8(ds_read16((lds_cbytes)(uintptr_t)koff[ks % kKOff] +
+                                              (kb + (ks / kKOff) * 256 + mt * (32 * A::kRowB))));
         // the first k-step starts from -m_ref (zero with the soft cap)
-        s_acc[mt] = mfma32(a, qt_op[ks], ks == 0 ? (kSoftCap ? f32x16{} : neg_mref) : s_acc[mt]);
+        s_acc[mt] = mfma32(a, qt_op[ks], ks == 0 ? (kFold ? neg_mref : f32x16{}) : s_acc[mt]);
       }
     }
   };
-  auto pv = [&](auto vst) __attribute__((always_inline)) {
+  // `vb`: the LDS byte offset of the tile's stage (a constant in the steady
+  // state, so it folds into the reads' immediate offsets)
+  auto pv = [&](uint32_t vb) __attribute__((always_inline)) {
+    if constexpr (!kV1) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      // k-step u: tokens 32(u/2) + 16(u%2) + {4h + r, 8 + 4h + r}
-      const int rb = decltype(vst)::value * kTileElems * 2 + (32 * (u >> 1) + 16 * (u & 1)) * 256;
+      for (int dt = 0; dt < kVOff; ++dt) asm volatile("v_xor_b32 %0, 32, %1" : "=v"(voff1[dt]) : "v"(voff0[dt]));
+    }
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        const s16x4 lo = ds_read_tr16((lds_cbytes)(uintptr_t)voff0[dt] + rb);
-        const s16x4 hi = ds_read_tr16((lds_cbytes)(uintptr_t)voff1[dt] + rb);
+    for (int u = 0; u < A::kU; ++u) {
+      // k-step u: tokens 16u + {4h + r, 8 + 4h + r}
+#pragma unroll
+      for (int dt = 0; dt < A::kDt; ++dt) {
+        const uint32_t rb = vb + 16 * u * A::kRowB + (dt / kVOff) * 256;
+        const s16x4 lo = ds_read_tr16((lds_cbytes)(uintptr_t)voff0[dt % kVOff] + rb);
+        const s16x4 hi = ds_read_tr16((lds_cbytes)(uintptr_t)voff1[dt % kVOff] + (rb + (kV1 ? 0 : 8 * A::kRowB)));
         const u32x2 lo2 = __builtin_bit_cast(u32x2, lo);
         const u32x2 hi2 = __builtin_bit_cast(u32x2, hi);
         const u32x4 a = {lo2[0], lo2[1], hi2[0], hi2[1]};
@@ -610,44 +687,53 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
       }
     }
   };
-  const float cap_s2 = kSoftCap ? soft_cap_s2(p.logit_scale, p.soft_cap) : 0.f;
-  const float cap_c = kSoftCap ? soft_cap_c(p.soft_cap) : 0.f;
+  // the cap's constants in scalar registers (the division's result is a vector one)
+  auto uniform = [](float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); };
+  const float cap_s2 = kSoftCap ? uniform(soft_cap_s2(p.logit_scale, p.soft_cap)) : 0.f;
+  const float cap_c = kSoftCap ? uniform(soft_cap_c(p.soft_cap)) : 0.f;
   const float cap_2c = 2.f * cap_c;
   auto softmax = [&](int t, auto&& between) __attribute__((always_inline)) {
-    const int j0 = t * kTileN;
+    const int j0 = t * kN;
     if constexpr (kSoftCap) {
       // capped logits relative to m_ref, as the uncapped S leaves the MFMAs
       const float cap_cm = cap_c - m_ref;
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
+      for (int mt = 0; mt < A::kMt; ++mt)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
           s_acc[mt][i] = soft_cap_log2_rel(s_acc[mt][i], cap_s2, cap_2c, cap_cm);
+    } else if constexpr (!kFold) {
+#pragma unroll
+      for (int mt = 0; mt < A::kMt; ++mt) s_acc[mt] = s_acc[mt] - m_ref;
     }
     // s_acc[mt][i] = S[row n][token j0 + 32mt + 8(i/4) + 4h + i%4]
     if (t >= n_free) {
       // token j = j0 + 4h + c is visible iff j < lk and j + kv_pos_off <=
       // qpos, i.e. iff c < lim: one compare and one select per element
       const int64_t hi = min((int64_t)lk, (int64_t)qpos - kv_pos_off + 1) - j0 - 4 * h;
-      int lim = (int)max((int64_t)0, min(hi, (int64_t)kTileN));
+      int lim = (int)max((int64_t)0, min(hi, (int64_t)kN));
       asm volatile("" : "+v"(lim));  // keeps the compares 32-bit (the compiler widens them otherwise)
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
+      for (int mt = 0; mt < A::kMt; ++mt)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
           s_acc[mt][i] = 32 * mt + 8 * (i >> 2) + (i & 3) < lim ? s_acc[mt][i] : -INFINITY;
     }
-    // four independent max3 chains (one per 16-token quarter)
-    float mq[4];
+    // independent max3 chains, one per 16 tokens
+    float mq[A::kU];
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
+    for (int q4 = 0; q4 < A::kU; ++q4) {
       const int mt = q4 >> 1, b0 = 8 * (q4 & 1);
       float m = __builtin_fmaxf(__builtin_fmaxf(s_acc[mt][b0], s_acc[mt][b0 + 1]), s_acc[mt][b0 + 2]);
       m = __builtin_fmaxf(__builtin_fmaxf(m, s_acc[mt][b0 + 3]), s_acc[mt][b0 + 4]);
       m = __builtin_fmaxf(__builtin_fmaxf(m, s_acc[mt][b0 + 5]), s_acc[mt][b0 + 6]);
       mq[q4] = __builtin_fmaxf(m, s_acc[mt][b0 + 7]);
     }
-    float mx = __builtin_fmaxf(__builtin_fmaxf(mq[0], mq[1]), __builtin_fmaxf(mq[2], mq[3]));
+#pragma unroll
+    for (int k = 1; k < A::kU; k *= 2)
+#pragma unroll
+      for (int q4 = 0; q4 < A::kU; q4 += 2 * k) mq[q4] = __builtin_fmaxf(mq[q4], mq[q4 + k]);
+    float mx = mq[0];
     mx = max_xor32(mx);  // log2 units: S is computed from the scaled Q (soft cap: capped logits)
     {
       // S is already relative to m_ref.  The first tile sets m_ref to the row
@@ -658,19 +744,21 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
         if (t != 0) {
           const float corr = fast_exp2(-d);
 #pragma unroll
-          for (int u = 0; u < 4; ++u) l_part[u] *= corr;
+          for (int u = 0; u < kL; ++u) l_part[u] *= corr;
 #pragma unroll
-          for (int dt = 0; dt < 4; ++dt) acc_o[dt] = acc_o[dt] * corr;
+          for (int dt = 0; dt < A::kDt; ++dt) acc_o[dt] = acc_o[dt] * corr;
         }
         m_ref += d;
+        if constexpr (kFold) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) neg_mref[i] = -m_ref;
+          for (int i = 0; i < 16; ++i) neg_mref[i] = -m_ref;
+        }
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) s_acc[mt] = s_acc[mt] - d;
+        for (int mt = 0; mt < A::kMt; ++mt) s_acc[mt] = s_acc[mt] - d;
       }
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < A::kU; ++u) {
       between(u);
       const int mt = u >> 1;
       const int base = 8 * (u & 1);
@@ -680,14 +768,15 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
         const float a = fast_exp2(s_acc[mt][base + 2 * e]);
         const float c = fast_exp2(s_acc[mt][base + 2 * e + 1]);
         w[e] = pack_bf16x2(a, c);
-        l_part[u] += a + c;
+        l_part[u % kL] += a + c;
       }
       // Materialise P here: otherwise the compiler sinks the exp work past
       // the barrier into the next MFMA segment, undoing the ping-pong.
       pt[u] = as_bf16x8(w);
       asm volatile("" : "+v"(pt[u]));
     }
-    asm volatile("" : "+v"(l_part[0]), "+v"(l_part[1]), "+v"(l_part[2]), "+v"(l_part[3]));
+    if constexpr (kL == 4) asm volatile("" : "+v"(l_part[0]), "+v"(l_part[1]), "+v"(l_part[2]), "+v"(l_part[3]));
+    else asm volatile("" : "+v"(l_part[0]), "+v"(l_part[1]));
   };
   auto barrier = [&]() __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
@@ -712,35 +801,35 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   const int ahead = grp_b ? 3 : 2;  // tile issued during SM(t) is t + ahead
   using T_ = std::true_type;
   using F_ = std::false_type;
-  // One M segment + one SM segment.  kPv / kQk say whether PV(t-1) / QK(t)
-  // exist (every iteration but the first and the last has both), so that the
-  // steady-state M segment is a single block the scheduler can interleave.
+  // One M segment + one SM segment.  kPv says whether PV(t-1) exists (every
+  // iteration but the first has both), so that the steady-state M segment is
+  // a single block the scheduler can interleave.
   int32_t page_next = 0;  // raw block-table entry of the next tile to load (aligned path)
   int nx_lp = 0, nx_r = 0;  // (aligned) table entry and in-page index of that tile
-  auto iteration = [&](int t, auto st, auto has_pv, auto has_qk) __attribute__((always_inline)) {
+  auto iteration = [&](int t, auto st, auto has_pv) __attribute__((always_inline)) {
     constexpr int s = decltype(st)::value;
     constexpr bool kPv = decltype(has_pv)::value;
-    constexpr bool kQk = decltype(has_qk)::value;
     using KS = std::integral_constant<int, s>;
-    using VS = std::integral_constant<int, (s + kStages - 1) % kStages>;
+    constexpr uint32_t kVb = (s + kStages - 1) % kStages * A::kStageB;
     // A wave with no row (past the last token of a sequence's last q tile)
     // skips its MFMA and softmax work in the steady-state iterations; its
     // tile loads, waits and barriers stay.  Under the part's power limit the
     // energy it saves goes to the other waves.
-    if (!(kPv && kQk) || wave_live) {
-    if constexpr (kPv) pv(VS{});
-    if constexpr (kQk) qk(KS{});
-    if constexpr (kPv && kQk) {
-      // 16 PV MFMAs (2 transposing V reads each) then 16 QK MFMAs (1 K read
-      // each): every read is issued kAheadMfma MFMAs before the MFMA it feeds.
-      constexpr int A = kAheadMfma;
-      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2 * A, 0);
+    if (!kPv || wave_live) {
+    if constexpr (kPv) pv(kVb);
+    qk(KS{});
+    if constexpr (kPv) {
+      // the PV MFMAs (2 transposing V reads each; 16 at head size 128) then
+      // the QK MFMAs (1 K read each; 16): every read is issued kAhead MFMAs
+      // before the MFMA it feeds.
+      constexpr int kAhead = A::kAhead, kPvN = A::kU * A::kDt, kAllN = kPvN + A::kMt * A::kKs;
+      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2 * kAhead, 0);
 #pragma unroll
-      for (int i = 1; i <= 32; ++i) {
-        const int next = i + A;  // MFMA whose operands are read now
+      for (int i = 1; i <= kAllN; ++i) {
+        const int next = i + kAhead;  // MFMA whose operands are read now
         __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
-        if (next <= 16) __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2, 0);
-        else if (next <= 32) __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
+        if (next <= kPvN) __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2, 0);
+        else if (next <= kAllN) __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
       }
     }
     }
@@ -751,32 +840,31 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
     // softmax has no branch around them and the waits count the same.
     const int ti = t + ahead;
     const int dstage = grp_b ? (s + 3) % kStages : (s + 2) % kStages;
-    TileAddrs ta;
-    if constexpr (kPv || kQk) ta = tile_addrs(ti * kTileN, page_next, nx_r);
-    if constexpr (kPaging == kPageTile && (kPv || kQk)) {  // for the next iteration: tile ti + 1
+    const TileAddrs ta = tile_addrs(ti * kN, page_next, nx_r);
+    if constexpr (kPaging == kPageTile) {  // for the next iteration: tile ti + 1
       if (++nx_r == tpp) {
         nx_r = 0;
         ++nx_lp;
       }
       page_next = page_raw_at(nx_lp);
-    } else if constexpr (kPaging == kPageWave && (kPv || kQk)) {
+    } else if constexpr (kPaging == kPageWave) {
       page_next = page_raw_at(wave_entry(ti + 1));
     }
-    // one DMA before each quarter of the softmax: a burst of them would
-    // stall on the address queue
+    // the tile's DMAs spread over the softmax (one before each quarter of a
+    // 64-token tile): a burst of them would stall on the address queue
     auto between = [&](int u) __attribute__((always_inline)) {
-      if constexpr (kPv || kQk) dma_issue(ta, u, dstage);
-    };
-    if constexpr (kQk) {
-      if (!kPv || wave_live) {
-        softmax(t, between);
+      if constexpr (A::kU >= kDmaPerTile) {
+        if (u % (A::kU / kDmaPerTile) == 0) dma_issue(ta, u / (A::kU / kDmaPerTile), dstage);
       } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) between(u);
+        for (int i = 0; i < kDmaPerTile / A::kU; ++i) dma_issue(ta, u * (kDmaPerTile / A::kU) + i, dstage);
       }
+    };
+    if (!kPv || wave_live) {
+      softmax(t, between);
     } else {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) between(u);
+      for (int u = 0; u < A::kU; ++u) between(u);
     }
     // this wave's share of tile t + ahead - 1 has landed: at most the loads of
     // tile t + ahead (issued above) may still be outstanding
@@ -793,8 +881,8 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   // barrier (which ends segment 0, i.e. before A's M(1) in segment 2).
   if (n_tiles > 0) {
     issue_tile_raw(0, raw_pre[0], 0);
-    issue_tile_raw(kTileN, raw_pre[1], 1);
-    if (grp_b) issue_tile_raw(2 * kTileN, raw_pre[2], 2);
+    issue_tile_raw(kN, raw_pre[1], 1);
+    if (grp_b) issue_tile_raw(2 * kN, raw_pre[2], 2);
   }
   // raw page id of the first tile the loop loads (tile `ahead`)
   if (kPaging == kPageTile && n_tiles > 0) {
@@ -818,27 +906,29 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
 
   // iterations t = 0 .. n_tiles: QK(0) alone, then PV(t-1) + QK(t), then
   // PV(n_tiles-1) alone.  Tile t sits in stage t % 4.
-  if (n_tiles == 0) {
-    iteration(0, S0{}, F_{}, F_{});
-  } else {
-    iteration(0, S0{}, F_{}, T_{});
-    int t = 1;
-    for (; t + 4 <= n_tiles; t += 4) {
-      iteration(t, S1{}, T_{}, T_{});
-      iteration(t + 1, S2{}, T_{}, T_{});
-      iteration(t + 2, S3{}, T_{}, T_{});
-      iteration(t + 3, S0{}, T_{}, T_{});
+  uint32_t v_last = 0;  // LDS byte offset of the last tile's stage
+  if (n_tiles > 0) {
+    iteration(0, S0{}, F_{});
+    for (int t = 1; t < n_tiles; ++t) {
+      iteration(t, S1{}, T_{});
+      v_last = A::kStageB;
+      if (++t == n_tiles) break;
+      iteration(t, S2{}, T_{});
+      v_last = 2 * A::kStageB;
+      if (++t == n_tiles) break;
+      iteration(t, S3{}, T_{});
+      v_last = 3 * A::kStageB;
+      if (++t == n_tiles) break;
+      iteration(t, S0{}, T_{});
+      v_last = 0;
     }
-    if (t < n_tiles) iteration(t, S1{}, T_{}, T_{});
-    if (t + 1 < n_tiles) iteration(t + 1, S2{}, T_{}, T_{});
-    if (t + 2 < n_tiles) iteration(t + 2, S3{}, T_{}, T_{});
-    switch (n_tiles & 3) {
-      case 0: iteration(n_tiles, S0{}, T_{}, F_{}); break;
-      case 1: iteration(n_tiles, S1{}, T_{}, F_{}); break;
-      case 2: iteration(n_tiles, S2{}, T_{}, F_{}); break;
-      default: iteration(n_tiles, S3{}, T_{}, F_{}); break;
-    }
+    // the last PV of a wave without rows runs too: its P is finite or zero
+    // and its O is never stored
+    pv(v_last);
   }
+  wait_vm_lgkm0<15>();
+  barrier();
+  barrier();
   if (!grp_b) barrier();
   wait_vm_lgkm0<0>();  // loads of tiles past the end may still be in flight
   PA_PHASE(ph3);
@@ -846,34 +936,37 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   // ---- epilogue.  acc_o[dt][i] of lane (n, h) holds row n, d = 32dt +
   // 8(i/4) + 4h + i%4: four consecutive d per i/4, i.e. the h-th half of
   // 16-byte chunk 4dt + i/4.  The normalised bf16 rows go to the wave's own
-  // blocks of stages 0 and 1 (every LDS read ended at the loop's last
-  // barrier, and this wave's own tile loads have landed), then out four
-  // whole 256-byte rows per store.
-  const float l_run = sum_xor32((l_part[0] + l_part[1]) + (l_part[2] + l_part[3]));
+  // blocks of the first kRowStages stages (every LDS read ended at the loop's
+  // last barrier, and this wave's own tile loads have landed),
+  // then out 1 KiB of whole rows per store.
+  const float l_run = kL == 4 ? sum_xor32((l_part[0] + l_part[1]) + (l_part[kL - 2] + l_part[kL - 1]))
+                              : sum_xor32(l_part[0] + l_part[1]);
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
 #pragma unroll
-  for (int dt = 0; dt < 4; ++dt)
+  for (int dt = 0; dt < A::kDt; ++dt)
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) {
+      if (4 * dt + q4 >= A::kChunks) continue;  // past the head size
       const f32x16& a = acc_o[dt];
       const int i = 4 * q4;
       const u32x2 v = {pack_bf16x2(a[i] * inv, a[i + 1] * inv), pack_bf16x2(a[i + 2] * inv, a[i + 3] * inv)};
       *reinterpret_cast<u32x2 __attribute__((address_space(3)))*>(
-          (uintptr_t)(piece(0, n >> 3) + 256 * (n & 7) + 16 * ((4 * dt + q4) ^ (n & 15)) + 8 * h)) = v;
+          (uintptr_t)(piece(0, n / A::kWaveRows) + A::kRowB * (n & (A::kWaveRows - 1)) +
+                      16 * ((4 * dt + q4) ^ A::qswz(n)) + 8 * h)) = v;
     }
   // A fresh lane index: the row arithmetic below repeats the Q loads'
   // expressions, which the compiler would otherwise carry through the loop.
   int lane_e = lane;
   asm volatile("" : "+v"(lane_e));
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = 4 * i + (lane_e >> 4);
-    const u32x4 v = ds_read16((lds_cbytes)(uintptr_t)(piece(0, r >> 3) + 256 * (r & 7) + 16 * (lane_e & 15)));
+  for (int i = 0; i < 32 / A::kBlkRows; ++i) {
+    const int r = A::kBlkRows * i + lane_e / A::kRowChunks;
+    const u32x4 v = ds_read16((lds_cbytes)(uintptr_t)(piece(0, i / A::kBlk) + 1024 * (i % A::kBlk) + 16 * lane_e));
     const int rw = wave * 32 + r;
     const int tk = (int)(((uint32_t)rw * gm) >> 24);
     const int hd = rw - tk * p.group;
-    const int c = (lane_e & 15) ^ (r & 15);
-    if (rw < p.tile_tokens * p.group && tok0 + tk < lq_rows)
+    const int c = (lane_e & (A::kRowChunks - 1)) ^ A::qswz(r);
+    if (c < A::kChunks && rw < p.tile_tokens * p.group && tok0 + tk < lq_rows)
       st16(p.out + (int64_t)(q0 + tok0 + tk) * p.o_ts + (int64_t)(kvh * p.group + hd) * p.o_hs + 8 * c, v);
   }
 #ifdef PA_PREFILL_PHASES
@@ -883,10 +976,61 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
 }
 
 // The work item numbered `bid`, resolved and run.
-template <bool kSoftCap, int kPaging>
+template <bool kSoftCap, int kPaging, int D = kPHeadDim>
 __device__ __forceinline__ void prefill_body(const PrefillParams& p, int bid) {
   PrefillWork w;
-  if (prefill_resolve(p, bid, w)) prefill_run<kSoftCap, kPaging>(p, w);
+  if (prefill_resolve(p, bid, w)) prefill_run<kSoftCap, kPaging, D>(p, w);
+}
+
+// Output rows the prefill items do not write, for 64 tokens t0 .. t0 + 63
+// (one wave): rows outside all sequences (before cu_q[0], from cu_q[batch]
+// on) and rows at offset >= max_seqlen_q inside their sequence (the
+// reference drops those too: its scatter only covers the first
+// max_seqlen_bucket rows, prefill...:384-388) are zeroed.  A lane checks one
+// token; the wave zeroes the rows it found, one after the other.
+template <int D>
+__device__ __forceinline__ void prefill_zero_rows(const PrefillParams& p, int64_t t0) {
+  const int lane = threadIdx.x & 63;
+  const int64_t t = t0 + lane;
+  const int32_t* cu_q = p.cu_q;
+  const int batch = p.batch;
+  bool zero = t < p.num_tokens;
+  if (zero && batch > 0 && t >= cu_q[0] && t < cu_q[batch]) {
+    // last b with cu_q[b] <= t
+    int lo = 0, hi = batch;  // invariant: cu_q[lo] <= t < cu_q[hi]
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (cu_q[mid] <= t) lo = mid;
+      else hi = mid;
+    }
+    zero = t - cu_q[lo] >= p.max_seqlen_q;
+  }
+  uint64_t todo = __ballot(zero);
+  const int chunks = p.num_heads * (D / 8);
+  while (todo) {
+    const int k = __ffsll((unsigned long long)todo) - 1;
+    todo &= todo - 1;
+    uint16_t* row = p.out + (t0 + k) * p.o_ts;
+    for (int c = lane; c < chunks; c += 64) {
+      const int hh = c / (D / 8);
+      st16(row + hh * p.o_hs + (c - hh * (D / 8)) * 8, u32x4{0, 0, 0, 0});
+    }
+  }
+}
+
+// kZero (launches without a work list): workgroups past the items zero the
+// rows no item writes, 512 tokens each, in place of a launch of their own.
+template <bool kSoftCap, int kPaging, bool kZero = false, int D = kPHeadDim>
+__global__ void __launch_bounds__(kThreads, 1) __attribute__((amdgpu_waves_per_eu(2 * PrefillDims<D, kSoftCap>::kWgs)))
+prefill_kernel(PrefillParams p) {
+  if constexpr (kZero) {
+    const int64_t items = (int64_t)p.n_qtiles * p.batch * p.num_kv_heads;
+    if (blockIdx.x >= items) {  // uniform over the workgroup
+      prefill_zero_rows<D>(p, ((int64_t)blockIdx.x - items) * kThreads + 64 * (threadIdx.x >> 6));
+      return;
+    }
+  }
+  prefill_body<kSoftCap, kPaging, D>(p, blockIdx.x);
 }
 
 // Tile paging of a launch (kPageLane / kPageTile / kPageWave).
