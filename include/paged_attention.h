@@ -183,6 +183,16 @@ int pa_prefill(const uint16_t* q, int64_t q_tok_stride, int64_t q_head_stride,
                uint16_t* out, int64_t out_tok_stride, int64_t out_head_stride,
                void* workspace, size_t workspace_bytes, void* stream);
 
+/* Workspace bytes with which pa_prefill also splits the items of a launch of
+ * few, long ones over their kv range and merges the parts (head_dim 128; other
+ * launches: pa_prefill_workspace_size).  A workspace between the two sizes
+ * runs unsplit.  pa_prefill_quant and pa_prefill_fp8 split when theirs is
+ * larger than pa_prefill_fp8_workspace_size by this minus
+ * pa_prefill_workspace_size.  0 for bad sizes; no counterpart in the
+ * reference, whose prefill grid is fixed. */
+size_t pa_prefill_split_workspace_size(int32_t batch, int32_t max_seqlen_q, int32_t num_heads, int32_t num_kv_heads,
+                                       int32_t head_dim, int32_t pages_per_seq, int32_t page_size);
+
 /* Workspace bytes of pa_prefill's work list (0 for bad sizes); no
  * counterpart in the reference, whose grid order is fixed. */
 size_t pa_prefill_workspace_size(int32_t batch, int32_t max_seqlen_q, int32_t num_heads,

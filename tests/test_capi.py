@@ -332,3 +332,20 @@ def test_generic_head_sizes_at_the_boundary():
         bad[9] = d
         assert lib.pa_kv_store_fp8(*bad) == -2
         assert "head_dim" in lib.pa_last_error().decode()
+
+
+def test_prefill_split_workspace_size():
+    lib = PKG._lib.load()
+    size = lib.pa_prefill_split_workspace_size
+    plan = lib.pa_prefill_workspace_size
+    slot = 4 * (256 * 128 + 2 * 256)     # f32 O, reference max and row sum of 256 rows
+    # 2 sequences x 512 rows of 64-token tiles: 16 pairs, 32 parts per kv head
+    # and as many again for rounding up (at most one per pair); 4 KiB of records
+    assert size(2, 512, 32, 8, 128, 64, 256) == 4096 + (32 + 16) * 8 * slot
+    assert size(1, 1, 32, 1, 128, 2048, 16) == 4096 + (256 + 1) * slot
+    for args in ((2, 512, 32, 8, 64, 64, 256),     # not head size 128
+                 (2, 512, 32, 8, 128, 5, 256),     # rows of 1 280 tokens: too short
+                 (64, 2048, 32, 8, 128, 64, 256),  # many items
+                 (0, 512, 32, 8, 128, 64, 256)):
+        assert size(*args) == plan(*args[:4])
+    assert size(2, 512, 33, 8, 128, 64, 256) == 0

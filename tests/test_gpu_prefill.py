@@ -425,3 +425,86 @@ def test_prefill_page_sizes_bit_identical(pkg, dev, prefix):
             assert err <= TOL
     for bs in (32, 48, 64, 256):
         assert np.array_equal(outs[bs], outs[16]), bs
+
+
+@pytest.mark.parametrize("prefix,new,h,hkv,bs,cap", [
+    ([1700, 2500, 0], [70, 1, 300], 32, 8, 16, None),     # 16-token pages, an item without a prefix
+    ([1700, 2500, 0], [70, 1, 300], 32, 8, 256, 20.0),    # soft cap
+    ([2000, 100], [65, 64], 64, 2, 24, None),             # G = 32, per-lane paging
+    ([3000], [1], 8, 1, 64, None),                        # one row, one kv head: 8 q rows, many parts
+    ([0], [1999], 16, 8, 16, None),                       # a fresh prompt: only its long items split
+    ([1600, 1, 0, 5], [0, 3, 128, 129], 12, 3, 32, None),  # a sequence without rows, 3 kv heads
+])
+def test_prefill_split_items(pkg, dev, prefix, new, h, hkv, bs, cap):
+    """Launches of few, long items split them over their kv range: the oracle,
+    and the unsplit launch (a workspace of the list's size only).  Both round
+    P to bf16 relative to their own reference max and O to bf16 once, O(1)
+    values: within the oracle's tolerance of each other."""
+    import torch
+    pb = wl.make_prefix_prefill(prefix, new, num_heads=h, num_kv_heads=hkv, page_size=bs,
+                                rng=np.random.default_rng(sum(new)), shared_prefix_tokens=0)
+    lib = pkg._lib.load()
+    plan = lib.pa_prefill_workspace_size(pb.batch, int(pb.max_seqlen_bucket), h, hkv)
+    split = lib.pa_prefill_split_workspace_size(pb.batch, int(pb.max_seqlen_bucket), h, hkv, 128,
+                                                pb.block_tables.shape[1], bs)
+    assert split > plan + 4 * 128 * 256
+    got, t = _prefill(pkg, dev, pb, seed=7, soft_cap=cap, use_seam=False)
+    args = (t["q"], t["kv_cache"][0].permute(2, 0, 1, 3), t["kv_cache"][1].permute(2, 0, 1, 3), t["block_tables"],
+            t["cu_seqlens_q"], t["slot_mapping"], t["input_positions"])
+    kw = dict(max_seqlen_bucket=pb.max_seqlen_bucket, cu_seqlens_k=t["cu_seqlens_k"], attn_logits_soft_cap=cap)
+    one = pkg.prefill_paged_attention(*args, workspace=torch.empty(plan, dtype=torch.uint8, device=dev), **kw)
+    assert np.abs(got - ora.bf16_to_f32(u16(one))).max() <= TOL
+    # a workspace full of NaNs (stale partials) changes nothing
+    ws = torch.full((split,), 255, dtype=torch.uint8, device=dev)
+    two = pkg.prefill_paged_attention(*args, workspace=ws, **kw)
+    assert np.array_equal(ora.bf16_to_f32(u16(two)), got)
+
+
+def test_prefill_split_rows_without_keys_and_rows_past_the_bucket(pkg, dev):
+    """Split launches: rows whose position precedes the first kv position,
+    rows past max_seqlen_bucket and rows outside every sequence are zeros."""
+    import torch
+    pb = wl.make_prefix_prefill([2500, 1800], [200, 90], num_heads=16, num_kv_heads=4, page_size=64,
+                                rng=np.random.default_rng(3), shared_prefix_tokens=0)
+    cu, first = pb.cu_seqlens_q, int(pb.input_positions[0])
+    pb.input_positions[40:60] = first - 2501 - np.arange(20)
+    got, t = _prefill(pkg, dev, pb, seed=8, use_seam=False)
+    assert not got[40:60].any() and got[60:int(cu[2])].any()
+    out = pkg.prefill_paged_attention(
+        t["q"], t["kv_cache"][0].permute(2, 0, 1, 3), t["kv_cache"][1].permute(2, 0, 1, 3), t["block_tables"],
+        t["cu_seqlens_q"], t["slot_mapping"], t["input_positions"], max_seqlen_bucket=128,
+        cu_seqlens_k=t["cu_seqlens_k"])
+    res = ora.bf16_to_f32(u16(out))
+    assert not res[128:200].any() and not res[int(cu[2]):].any()
+    keep = np.r_[0:128, 200:290]
+    assert np.abs(res[keep] - got[keep]).max() <= TOL
+
+
+def test_prefill_split_graph_replay(pkg, dev):
+    """A captured split launch, replayed with eager work between, equals the
+    eager result every time."""
+    import torch
+    pb = wl.make_prefix_prefill([4000, 300], [100, 40], num_heads=32, num_kv_heads=8, page_size=16,
+                                rng=np.random.default_rng(4), shared_prefix_tokens=0)
+    t = wl.materialize_prefill(pb, 9, dev, fill_pool=True)
+    out = torch.empty_like(t["q"])
+    call = lambda o: pkg.prefill_paged_attention(  # noqa: E731
+        t["q"], t["kv_cache"][0].permute(2, 0, 1, 3), t["kv_cache"][1].permute(2, 0, 1, 3), t["block_tables"],
+        t["cu_seqlens_q"], t["slot_mapping"], t["input_positions"], max_seqlen_bucket=pb.max_seqlen_bucket,
+        cu_seqlens_k=t["cu_seqlens_k"], out=o)
+    want = call(torch.empty_like(out)).clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(out)
+    torch.cuda.current_stream().wait_stream(side)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        call(out)
+    for _ in range(4):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+        call(torch.empty_like(out))
+        torch.cuda.synchronize()

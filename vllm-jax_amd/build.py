@@ -27,7 +27,7 @@ PHASES_LIB_PATH = os.path.join(os.path.dirname(PKG_DIR), "libpaged_attention_pha
 ARCH = "gfx950"
 
 SOURCES = ["pa_errors.cpp", "block_manager.cpp", "kv_store.hip", "decode.hip", "prefill.hip", "prefill_heads.hip",
-           "qk_norm_rope.hip", "mixed.hip", "any_head.hip"]
+           "prefill_split.hip", "qk_norm_rope.hip", "mixed.hip", "any_head.hip"]
 PHASES_SOURCES = ["pa_errors.cpp", "prefill.hip", "any_head.hip"]  # any_head: the head-size check of the quantized entries
 
 # Packed-FP32 VALU forms are disabled for every device compile: the build

@@ -5,6 +5,7 @@
 
 #include "any_head.h"
 #include "prefill_impl.h"
+#include "prefill_split.h"
 
 namespace pa {
 
@@ -467,6 +468,13 @@ static int prefill_launch(const char* name, const uint16_t* q, int64_t q_tok_str
   // the work list needs every sequence's geometry in the planner's LDS
   const bool planned = workspace && batch > 0 && max_seqlen_q > 0 && batch <= kPlanMaxBatch &&
                        items >= kPrefillPlanMinItems;
+#ifndef PA_PREFILL_PHASES
+  if (workspace && !planned && batch > 0 && prefill_splits(prm)) {  // few items: split the long ones if the workspace holds their partials
+    const size_t split = prefill_split_bytes(batch, prm.n_qtiles, num_kv_heads, (int64_t)pages_per_seq * page_size);
+    if (split && workspace_bytes >= split)
+      return prefill_split_launch(name, prm, prefill_paging(page_size, slot_stride), workspace, s);
+  }
+#endif
   int32_t* plan = planned ? reinterpret_cast<int32_t*>(workspace) : nullptr;
   if (planned) {  // the list and the zero rows, ahead of the prefill
     const int64_t zero_blocks = (num_tokens + kPrepThreads / 64 - 1) / (kPrepThreads / 64) + 1;
@@ -516,6 +524,18 @@ extern "C" size_t pa_prefill_workspace_size(int32_t batch, int32_t max_seqlen_q,
   const int64_t pairs = (int64_t)batch * ((max_seqlen_q + tile_tokens - 1) / tile_tokens);
   return (size_t)(kPlanHeader + 8 * pairs) * sizeof(int32_t);
 }
+
+#ifndef PA_PREFILL_PHASES
+extern "C" size_t pa_prefill_split_workspace_size(int32_t batch, int32_t max_seqlen_q, int32_t num_heads,
+                                                  int32_t num_kv_heads, int32_t head_dim, int32_t pages_per_seq,
+                                                  int32_t page_size) {
+  const size_t plan = pa_prefill_workspace_size(batch, max_seqlen_q, num_heads, num_kv_heads);
+  if (!plan || head_dim != kPHeadDim || pages_per_seq < 0 || page_size <= 0) return plan;
+  const int32_t tile_tokens = kRows / (num_heads / num_kv_heads);
+  return std::max(plan, prefill_split_bytes(batch, (int32_t)(((int64_t)max_seqlen_q + tile_tokens - 1) / tile_tokens),
+                                            num_kv_heads, (int64_t)pages_per_seq * page_size));
+}
+#endif
 
 extern "C" int pa_prefill(const uint16_t* q, int64_t q_tok_stride, int64_t q_head_stride,
                           const uint16_t* k_cache, const uint16_t* v_cache,
@@ -632,7 +652,8 @@ static int prefill_quant(const char* name, int32_t code, const uint16_t* q, int6
                         pages_per_seq, cu_seqlens_q, cu_seqlens_k, input_positions, batch, num_tokens, max_seqlen_q,
                         num_heads, num_kv_heads, head_dim, scale, soft_cap, out, out_tok_stride, out_head_stride,
                         (char*)workspace + fp8_widened_bytes(batch, pages_per_seq, page_size, num_kv_heads, head_dim),
-                        need - fp8_widened_bytes(batch, pages_per_seq, page_size, num_kv_heads, head_dim), stream);
+                        workspace_bytes - fp8_widened_bytes(batch, pages_per_seq, page_size, num_kv_heads, head_dim),
+                        stream);
 }
 
 extern "C" int pa_prefill_quant(int32_t code_type, const uint16_t* q, int64_t q_tok_stride, int64_t q_head_stride,

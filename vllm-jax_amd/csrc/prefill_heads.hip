@@ -6,8 +6,8 @@
 // come straight into a four-stage LDS ring and one wave of a SIMD feeds the
 // matrix cores while the other takes its softmax.  16 sequences of 1000 to
 // 3000 tokens, 32 / 8 heads, generic -> this (one MI355X): 64 391 -> 351 us,
-// 96 522 -> 503 (soft cap 852 -> 636), 256 1920 -> 1282 (soft cap 2028 ->
-// 1298); one sequence of 32768 tokens: 64 4.82 -> 4.31 ms, 256 25.1 -> 16.7.
+// 96 522 -> 511 (soft cap 852 -> 653), 256 1927 -> 1316 (soft cap 2037 ->
+// 1326); one sequence of 32768 tokens: 64 4.82 -> 4.31 ms, 256 25.1 -> 16.7.
 // Bound by the softmax's VALU work at 64, by MFMA and LDS reads at 256, and
 // by the ~7 us an item spends outside its loop at these lengths.  80 gained
 // nothing (492 us against 478, its generic kernel also fits two workgroups a

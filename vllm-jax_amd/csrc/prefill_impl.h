@@ -83,6 +83,10 @@ struct PrefillParams {
   // Work list (may be null): plan[0] = number of (sequence, q tile) pairs with
   // rows, PrefillPair records from int kPlanHeader on, most kv tiles first.
   const int32_t* plan;
+  // Launches that split items over the kv range (prefill_split.hip): a record
+  // (parts, first slot, q0, rows) per (sequence, q tile) pair, and the partials.
+  int32_t* split;
+  float* parts;
   // With the work list and num_kv_heads % 8 == 0: the counters of the eight
   // XCDs' pools (plan + 8 .. plan + 15, zeroed by the list builder), see
   // prefill_kernel_pooled; null otherwise.
@@ -146,9 +150,6 @@ struct PrefillDims {
   // The QK accumulators start from -m_ref where the registers allow it (16
   // of them); elsewhere the reference is subtracted from S.
   static constexpr bool kFoldRef = kRowB == 256 && kWgs == 1;
-  // MFMAs between an LDS read and the MFMA it feeds (at 512-byte rows one
-  // operand's registers fewer: four spilled an address in the loop)
-  static constexpr int kAhead = kRowB < 512 ? kAheadMfma : 3;
   // Chunk swizzle of tile row r (XORed into the chunk index, low 4 bits of
   // r): 16 rows' reads of one chunk and a transposing read's 4 rows x 64
   // bytes both land on distinct banks.
@@ -357,9 +358,25 @@ __device__ __forceinline__ bool prefill_resolve(const PrefillParams& p, int bid,
   return true;
 }
 
-// One prefill work item, run by a whole 512-thread workgroup.
-template <bool kSoftCap, int kPaging, int D = kPHeadDim>
-__device__ __forceinline__ void prefill_run(const PrefillParams& p, const PrefillWork& w) {
+// The kv tiles [lo, hi) of an item, for launches that split items over the kv
+// range: the workgroup leaves its unnormalised O (f32), reference max and row
+// sums in partial `slot`, or finishes the item itself (slot < 0: all tiles).
+struct PrefillPart {
+  int lo, hi, slot;
+};
+// A partial's O: 16 bytes (four d) per lane and (32-row block, chunk), as the
+// accumulators hold them; then (reference max, row sum) of its 256 rows.
+template <int D>
+constexpr int kPartO = kRows * ((D + 31) / 32 * 32);  // floats
+template <int D>
+constexpr int kPartFloats = kPartO<D> + 2 * kRows;
+
+// One prefill work item (kSplit: one part of it), run by a whole 512-thread
+// workgroup.
+template <bool kSoftCap, int kPaging, int D = kPHeadDim, bool kSplit = false>
+__device__ __forceinline__ void prefill_run(const PrefillParams& p, const PrefillWork& w,
+                                            const PrefillPart& part = {0, INT_MAX, -1}) {
+  const int base = kSplit ? part.lo : 0;  // first tile; the loop counts from it
   using A = PrefillDims<D, kSoftCap>;
   constexpr int kN = A::kN;
   constexpr bool kAligned = kPaging != kPageLane;  // scalar page bases
@@ -436,7 +453,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
           (const __attribute__((address_space(4))) int32_t*)(p.block_tables + (int64_t)b * p.bt_stride);
 #pragma unroll
       for (int i = 0; i < 3; ++i)
-        raw_pre[i] = c[min(kPaging == kPageWave ? wave_entry(i) : i * kN / p.page_size, p.pages_per_seq - 1)];
+        raw_pre[i] = c[min(kPaging == kPageWave ? wave_entry(base + i) : (base + i) * kN / p.page_size, p.pages_per_seq - 1)];
     }
   }
 
@@ -489,11 +506,12 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   // kv index j is visible to some row iff j < lk and j + kv_pos_off <= qpos_max
   const int64_t kv_hi64 = min((int64_t)lk, (int64_t)qpos_max - kv_pos_off + 1);
   const int kv_hi = kv_hi64 < 0 ? 0 : (int)kv_hi64;
-  const int n_tiles = (kv_hi + kN - 1) / kN;
+  int n_tiles = (kv_hi + kN - 1) / kN;
+  if constexpr (kSplit) n_tiles = max(0, min(n_tiles, part.hi) - base);
   PA_PHASE(ph1);
   // tiles [0, n_free) need no mask: every token is < lk and visible to every row
   const int64_t free_hi = min((int64_t)lk, (int64_t)qpos_min - kv_pos_off + 1);
-  const int n_free = free_hi < 0 ? 0 : (int)(free_hi / kN);
+  const int n_free = (free_hi < 0 ? 0 : (int)(free_hi / kN)) - base;
 
   // ---- direct global->LDS tile loader.  A tile is kWaves * kBlk blocks of
   // 1 KiB (kBlkRows rows each); wave w fills blocks kBlk*w .. kBlk*w + kBlk-1 of K
@@ -693,7 +711,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   const float cap_c = kSoftCap ? uniform(soft_cap_c(p.soft_cap)) : 0.f;
   const float cap_2c = 2.f * cap_c;
   auto softmax = [&](int t, auto&& between) __attribute__((always_inline)) {
-    const int j0 = t * kN;
+    const int j0 = (base + t) * kN;
     if constexpr (kSoftCap) {
       // capped logits relative to m_ref, as the uncapped S leaves the MFMAs
       const float cap_cm = cap_c - m_ref;
@@ -822,7 +840,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
       // the PV MFMAs (2 transposing V reads each; 16 at head size 128) then
       // the QK MFMAs (1 K read each; 16): every read is issued kAhead MFMAs
       // before the MFMA it feeds.
-      constexpr int kAhead = A::kAhead, kPvN = A::kU * A::kDt, kAllN = kPvN + A::kMt * A::kKs;
+      constexpr int kAhead = kAheadMfma, kPvN = A::kU * A::kDt, kAllN = kPvN + A::kMt * A::kKs;
       __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2 * kAhead, 0);
 #pragma unroll
       for (int i = 1; i <= kAllN; ++i) {
@@ -840,7 +858,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
     // softmax has no branch around them and the waits count the same.
     const int ti = t + ahead;
     const int dstage = grp_b ? (s + 3) % kStages : (s + 2) % kStages;
-    const TileAddrs ta = tile_addrs(ti * kN, page_next, nx_r);
+    const TileAddrs ta = tile_addrs((base + ti) * kN, page_next, nx_r);
     if constexpr (kPaging == kPageTile) {  // for the next iteration: tile ti + 1
       if (++nx_r == tpp) {
         nx_r = 0;
@@ -848,7 +866,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
       }
       page_next = page_raw_at(nx_lp);
     } else if constexpr (kPaging == kPageWave) {
-      page_next = page_raw_at(wave_entry(ti + 1));
+      page_next = page_raw_at(wave_entry(base + ti + 1));
     }
     // the tile's DMAs spread over the softmax (one before each quarter of a
     // 64-token tile): a burst of them would stall on the address queue
@@ -880,17 +898,17 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   // tile 0 before the first barrier; B also waits for tile 1 before its idle
   // barrier (which ends segment 0, i.e. before A's M(1) in segment 2).
   if (n_tiles > 0) {
-    issue_tile_raw(0, raw_pre[0], 0);
-    issue_tile_raw(kN, raw_pre[1], 1);
-    if (grp_b) issue_tile_raw(2 * kN, raw_pre[2], 2);
+    issue_tile_raw(base * kN, raw_pre[0], 0);
+    issue_tile_raw((base + 1) * kN, raw_pre[1], 1);
+    if (grp_b) issue_tile_raw((base + 2) * kN, raw_pre[2], 2);
   }
   // raw page id of the first tile the loop loads (tile `ahead`)
   if (kPaging == kPageTile && n_tiles > 0) {
-    nx_lp = ahead / tpp;
-    nx_r = ahead - nx_lp * tpp;
+    nx_lp = (base + ahead) / tpp;
+    nx_r = base + ahead - nx_lp * tpp;
     page_next = page_raw_at(nx_lp);
   } else if (kPaging == kPageWave && n_tiles > 0) {
-    page_next = page_raw_at(wave_entry(ahead));
+    page_next = page_raw_at(wave_entry(base + ahead));
   }
   const int issued = n_tiles > 0 ? (grp_b ? 3 : 2) : 0;
   if (issued == 3) wait_vm_lgkm0<2 * kDmaPerTile>();
@@ -941,6 +959,23 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, const Prefil
   // then out 1 KiB of whole rows per store.
   const float l_run = kL == 4 ? sum_xor32((l_part[0] + l_part[1]) + (l_part[kL - 2] + l_part[kL - 1]))
                               : sum_xor32(l_part[0] + l_part[1]);
+  if constexpr (kSplit) {
+    if (part.slot >= 0) {  // uniform over the workgroup
+      float* dst = p.parts + (int64_t)part.slot * kPartFloats<D>;
+#pragma unroll
+      for (int dt = 0; dt < A::kDt; ++dt)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const f32x16& a = acc_o[dt];
+          *reinterpret_cast<f32x4*>(dst + 4 * (((wave * A::kDt + dt) * 4 + q4) * 64 + lane)) =
+              f32x4{a[4 * q4], a[4 * q4 + 1], a[4 * q4 + 2], a[4 * q4 + 3]};
+        }
+      // a row that saw no key here carries no weight, whatever its reference
+      if (h == 0)
+        *reinterpret_cast<f32x2*>(dst + kPartO<D> + 2 * row) = f32x2{l_run > 0.f ? m_ref : -INFINITY, l_run};
+      return;
+    }
+  }
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
 #pragma unroll
   for (int dt = 0; dt < A::kDt; ++dt)

@@ -1,0 +1,238 @@
+// Prefill of few, long items: split over the kv range, then merged.
+//
+// One (q tile, sequence, kv head) item per workgroup leaves most of the chip
+// idle when there are few of them: two new turns of 128 to 400 tokens behind
+// 6 000 to 15 000 cached ones are 72 items of up to 240 kv tiles on 256 CUs.
+// Here every workgroup first counts the launch's kv tiles (one thread per
+// (sequence, q tile) pair, as prefill_plan estimates them), finds a part
+// length with which the parts fill the chip once, and runs one part of one
+// item, longest parts first.  A part leaves its unnormalised O, reference max
+// and row sums in f32; prefill_split_merge_kernel adds the parts up.  That
+// call: 226 us unsplit, 89.7 + 8.0 us so (131 with parts of an even share,
+// whose 288 parts took two rounds).  What is left: about 1.1 us a tile and 10
+// us around the loop, and 32 MB of partials written and read.
+#include <algorithm>
+#include <climits>
+
+#include "prefill_impl.h"
+#include "prefill_split.h"
+
+namespace pa {
+namespace {
+
+constexpr int kSplitCUs = 256;
+// Pairs the in-kernel count takes: each of up to 256 threads compares its pair
+// with all others.
+constexpr int kSplitMaxPairs = 256;
+// No part below this many tiles is made: a part costs about 7 us outside its
+// loop, and a tile about 1 us.
+constexpr int kSplitMinTiles = 8;
+// Shortest table span (in kv tiles) that is worth the merge launch.
+constexpr int kSplitMinSpan = 24;
+// Bound on the items (pairs with rows x kv heads) of a launch that splits.
+// From a CU's worth on the parts need a second round, each with its own fixed
+// cost, and the merge: one 1 999-token prompt (256 items of 1 to 32 tiles,
+// Qwen3-8B heads) took 52 us unsplit and 55 + 10 us split.
+constexpr int64_t kSplitMaxItems = kSplitCUs;
+// Largest grid (n_qtiles x batch x kv heads) that is looked at.
+constexpr int64_t kSplitMaxGrid = 1024;
+
+// Parts and slots of a launch: sum over pairs of ceil(tiles / L) with L at
+// least an even share, tiles * kv heads / kSplitCUs, is at most kSplitCUs / kv
+// heads + pairs; only split pairs (two parts or more, so longer than L, so at
+// most kSplitCUs / kv heads of them) take slots.
+int64_t split_max_parts(int64_t pairs, int32_t hkv) { return kSplitCUs / hkv + pairs; }
+int64_t split_max_slots(int64_t pairs, int32_t hkv) {
+  const int64_t share = kSplitCUs / hkv;
+  return (share + (pairs < share ? pairs : share)) * hkv;
+}
+constexpr size_t kSplitHeader = kSplitMaxPairs * 4 * sizeof(int32_t);
+
+template <bool kSoftCap, int kPaging>
+__global__ void __launch_bounds__(kThreads, 1)
+prefill_split_kernel(PrefillParams p, int grid_parts) {
+  if ((int)blockIdx.x >= grid_parts) {  // uniform over the workgroup
+    prefill_zero_rows<kPHeadDim>(p, ((int64_t)blockIdx.x - grid_parts) * kThreads + 64 * (threadIdx.x >> 6));
+    return;
+  }
+  __shared__ unsigned long long s_total;
+  __shared__ int32_t s_tiles[kSplitMaxPairs], s_size[kSplitMaxPairs], s_parts[kSplitMaxPairs];
+  __shared__ int32_t s_work[12];
+  const int tid = threadIdx.x;
+  const int hkv = p.num_kv_heads;
+  const int nq = p.n_qtiles;
+  const int pairs = p.batch * nq;
+  const int mine = blockIdx.x / hkv;  // part of the launch's list; kv head bid % hkv (one XCD per head)
+  if (tid == 0) {
+    s_total = 0;
+    s_work[0] = -1;
+  }
+  __syncthreads();
+  int4 g = {};
+  int tiles = -1, b = 0, qt = 0;
+  if (tid < pairs) {
+    int lag;
+    b = tid / nq;
+    qt = tid - b * nq;
+    prefill_seq_geometry(p, b, g, lag);
+    tiles = prefill_pair_tiles(g, lag, qt, p.tile_tokens);  // -1: no rows
+    if (tiles > 0) atomicAdd(&s_total, (unsigned long long)tiles);
+    s_tiles[tid] = tiles;
+  }
+  __syncthreads();
+  // The part length: an even share of the launch's tiles leaves more parts
+  // than CUs (every pair rounds up), so lane k of each wave counts the parts
+  // at a share times 1 + k / 16 and the shortest length that fits one round
+  // is taken (the even share if none does).
+  const int64_t share = ((int64_t)s_total * hkv + kSplitCUs - 1) / kSplitCUs;
+  const int lane = tid & 63;
+  const int64_t least = max((int64_t)kSplitMinTiles, share);
+  const int cand = (int)min(least + least * lane / 16, (int64_t)INT_MAX);
+  const float inv = 1.f / (float)cand;
+  float count = 0.f;
+  for (int j = 0; j < pairs; ++j) {
+    const float tj = (float)s_tiles[j];
+    count += tj < 0.f ? 0.f : fmaxf(1.f, ceilf(tj * inv));
+  }
+  const uint64_t fits = __ballot(count * (float)hkv <= (float)kSplitCUs);
+  const int len = __shfl(cand, fits ? __ffsll((unsigned long long)fits) - 1 : 0);
+  const int parts = tiles < 0 ? 0 : max(1, (int)(((int64_t)tiles + len - 1) / len));
+  const int size = parts ? (tiles + parts - 1) / parts : -1;
+  if (tid < kSplitMaxPairs) {
+    s_size[tid] = size;
+    s_parts[tid] = parts;
+  }
+  __syncthreads();
+  if (tid < pairs && parts) {
+    int at = 0, slot = 0;  // parts listed before this pair's, and partials
+    for (int j = 0; j < pairs; ++j) {
+      const int sj = s_size[j], pj = s_parts[j];
+      const bool before = sj > size || (sj == size && j < tid);
+      at += before ? pj : 0;
+      slot += before && pj > 1 ? pj : 0;
+    }
+    if (mine >= at && mine < at + parts) {
+      const int k = mine - at;
+      s_work[0] = b;
+      s_work[1] = qt;
+      s_work[2] = g.x;
+      s_work[3] = g.y;
+      s_work[4] = g.z;
+      s_work[5] = g.w;
+      s_work[6] = (int)((int64_t)tiles * k / parts);
+      s_work[7] = k + 1 == parts ? INT_MAX : (int)((int64_t)tiles * (k + 1) / parts);
+      s_work[8] = parts > 1 ? (slot + k) * hkv : -1;
+    }
+    if (blockIdx.x == 0) {  // for the merge
+      st16(p.split + 4 * tid, u32x4{(uint32_t)parts, (uint32_t)(slot * hkv), (uint32_t)g.x, (uint32_t)g.y});
+    }
+  } else if (tid < pairs && blockIdx.x == 0) {
+    p.split[4 * tid] = 0;
+  }
+  __syncthreads();
+  auto work = [&](int i) { return __builtin_amdgcn_readfirstlane(s_work[i]); };
+  PrefillWork w;
+  w.b = work(0);
+  if (w.b < 0) return;  // past the list; uniform over the workgroup
+  w.qt = work(1);
+  w.kvh = (int)blockIdx.x - mine * hkv;
+  w.q0 = work(2);
+  w.lq_rows = work(3);
+  w.lk = work(4);
+  w.kv_pos_off = work(5);
+  PrefillPart part;
+  part.lo = work(6);
+  part.hi = work(7);
+  part.slot = work(8);
+  if (part.slot >= 0) part.slot += w.kvh;
+  prefill_run<kSoftCap, kPaging, kPHeadDim, true>(p, w, part);
+}
+
+// out = sum_k o_k 2^(m_k - M) / sum_k l_k 2^(m_k - M) over an item's parts k,
+// M their largest reference max.
+// One workgroup per (pair, kv head, 32-row block), one wave per 32 d: the
+// lanes hold what the part's accumulators held.
+__global__ void __launch_bounds__(256)
+prefill_split_merge_kernel(PrefillParams p) {
+  const int hkv = p.num_kv_heads;
+  const int item = blockIdx.x / kWaves;
+  const int block = blockIdx.x - item * kWaves;
+  const int pair = item / hkv;
+  const int kvh = item - pair * hkv;
+  const int4 rec = *reinterpret_cast<const int4*>(p.split + 4 * pair);  // parts, first slot, q0, rows
+  const int parts = rec.x;
+  if (parts < 2) return;
+  const float* src = p.parts + (int64_t)(rec.y + kvh) * kPartFloats<kPHeadDim>;
+  const int64_t step = (int64_t)hkv * kPartFloats<kPHeadDim>;
+  const int lane = threadIdx.x & 63;
+  const int dt = threadIdx.x >> 6;
+  const int n = lane & 31, h = lane >> 5;
+  const int row = 32 * block + n;
+  const int rtok = (pair - pair / p.n_qtiles * p.n_qtiles) * p.tile_tokens + row / p.group;
+  const float* ml = src + kPartO<kPHeadDim> + 2 * row;
+  const float* po = src + 4 * ((block * 4 + dt) * 4 * 64 + lane);
+  f32x4 o[4] = {};
+  float m_run = -INFINITY, lsum = 0.f;
+  // the sums follow a running max, so that no load waits for another part's
+#pragma unroll 4
+  for (int k = 0; k < parts; ++k) {
+    const f32x2 v = *reinterpret_cast<const f32x2*>(ml + k * step);
+    const float m_new = fmaxf(m_run, v[0]);
+    const float ms = m_new == -INFINITY ? 0.f : m_new;
+    const float old = fast_exp2(m_run - ms), wgt = fast_exp2(v[0] - ms);
+    m_run = m_new;
+    lsum = lsum * old + v[1] * wgt;
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4)
+      o[q4] = o[q4] * old + *reinterpret_cast<const f32x4*>(po + k * step + 256 * q4) * wgt;
+  }
+  if (row >= p.tile_tokens * p.group || rtok >= rec.w) return;
+  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;  // rows that see no key are zeros
+  uint16_t* orow = p.out + (int64_t)(rec.z + rtok) * p.o_ts +
+                   (int64_t)(kvh * p.group + row - row / p.group * p.group) * p.o_hs + 32 * dt + 4 * h;
+#pragma unroll
+  for (int q4 = 0; q4 < 4; ++q4)
+    *reinterpret_cast<u32x2*>(orow + 8 * q4) =
+        u32x2{pack_bf16x2(o[q4][0] * inv, o[q4][1] * inv), pack_bf16x2(o[q4][2] * inv, o[q4][3] * inv)};
+}
+
+}  // namespace
+
+size_t prefill_split_bytes(int32_t batch, int32_t n_qtiles, int32_t num_kv_heads, int64_t span) {
+  const int64_t pairs = (int64_t)batch * n_qtiles;
+  if (pairs <= 0 || pairs > kSplitMaxPairs || pairs * num_kv_heads > kSplitMaxGrid ||
+      span < (int64_t)kSplitMinSpan * kTileN)
+    return 0;
+  return kSplitHeader + (size_t)split_max_slots(pairs, num_kv_heads) * kPartFloats<kPHeadDim> * sizeof(float);
+}
+
+bool prefill_splits(const PrefillParams& p) {
+  // pairs with rows: a sequence of n tokens has ceil(n / tile_tokens)
+  const int64_t live = std::min<int64_t>((int64_t)p.batch * p.n_qtiles, p.num_tokens / p.tile_tokens + p.batch);
+  return live * p.num_kv_heads < kSplitMaxItems;
+}
+
+int prefill_split_launch(const char* name, const PrefillParams& prm, int paging, void* workspace, hipStream_t s) {
+  PrefillParams p = prm;
+  p.split = reinterpret_cast<int32_t*>(workspace);
+  p.parts = reinterpret_cast<float*>((char*)workspace + kSplitHeader);
+  const int64_t pairs = (int64_t)p.batch * p.n_qtiles;
+  const int grid_parts = (int)(split_max_parts(pairs, p.num_kv_heads) * p.num_kv_heads);
+  // workgroups past the parts zero the rows no item writes, 512 tokens each
+  const int64_t blocks = grid_parts + ((int64_t)p.num_tokens + kThreads - 1) / kThreads;
+  const dim3 grid((unsigned)blocks), blk(kThreads);
+  auto launch = [&](auto cap) {
+    constexpr bool kCap = decltype(cap)::value;
+    if (paging == kPageTile) prefill_split_kernel<kCap, kPageTile><<<grid, blk, 0, s>>>(p, grid_parts);
+    else if (paging == kPageWave) prefill_split_kernel<kCap, kPageWave><<<grid, blk, 0, s>>>(p, grid_parts);
+    else prefill_split_kernel<kCap, kPageLane><<<grid, blk, 0, s>>>(p, grid_parts);
+  };
+  if (p.soft_cap > 0.f) launch(std::true_type{});
+  else launch(std::false_type{});
+  const int rc = launch_status(name);
+  if (rc) return rc;
+  prefill_split_merge_kernel<<<dim3((unsigned)(pairs * p.num_kv_heads * kWaves)), dim3(256), 0, s>>>(p);
+  return launch_status(name);
+}
+
+}  // namespace pa

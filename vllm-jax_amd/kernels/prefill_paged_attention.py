@@ -59,7 +59,9 @@ def prefill_paged_attention(
       * ``scale`` -- logit scale (default: bf16(1/sqrt(d)) as prefill...:60);
       * ``out`` -- preallocated output;
       * ``workspace`` -- device bytes for the work list that orders the
-        kernel's items by kv length (``pa_prefill_workspace_size``) and, for
+        kernel's items by kv length (``pa_prefill_workspace_size``; with
+        ``pa_prefill_split_workspace_size`` bytes a launch of few, long items
+        also splits them over their kv range) and, for
         quantized pages (float8 e4m3fn codes, or int8 / uint8 integers, with
         float32 ``[Hkv, NB, BS]`` per-token scales), the pages widened to bf16 ahead of it
         (``pa_prefill_fp8_workspace_size``); allocated when absent or too small.
@@ -117,13 +119,16 @@ def prefill_paged_attention(
     soft_cap = 0.0 if attn_logits_soft_cap is None else float(attn_logits_soft_cap)
     ps, ss, hs = pages_strides(k_pages)
     lib = _lib.load()
+    need = int(lib.pa_prefill_workspace_size(batch, int(max_seqlen_bucket), num_heads, num_kv_heads))
+    extra = 0  # bytes of the widened pages
     if quantized:
-        need = int(lib.pa_prefill_fp8_workspace_size(batch, pages_per_sequence, page_size, num_kv_heads, head_dim,
-                                                     int(max_seqlen_bucket), num_heads))
-    else:
-        need = int(lib.pa_prefill_workspace_size(batch, int(max_seqlen_bucket), num_heads, num_kv_heads))
-    if workspace is None or workspace.numel() * workspace.element_size() < need:
-        workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
+        extra = int(lib.pa_prefill_fp8_workspace_size(batch, pages_per_sequence, page_size, num_kv_heads, head_dim,
+                                                      int(max_seqlen_bucket), num_heads)) - need
+    if workspace is None or workspace.numel() * workspace.element_size() < need + extra:
+        # our own: with room for the parts of a launch that splits its items
+        need = int(lib.pa_prefill_split_workspace_size(batch, int(max_seqlen_bucket), num_heads, num_kv_heads,
+                                                       head_dim, pages_per_sequence, page_size))
+        workspace = torch.empty(max(need + extra, 1), dtype=torch.uint8, device=q.device)
     ws_bytes = workspace.numel() * workspace.element_size()
     if quantized:
         _lib.call(
