@@ -116,3 +116,24 @@ def test_kv_store_duplicate_slot_check(pkg, dev, monkeypatch):
     monkeypatch.delenv("PA_CHECK_SLOTS")
     pkg.update_kv_cache(cache, sm, k, v)
     torch.cuda.synchronize()
+
+
+def test_attention_stored_takes_pools_and_pairs_of_halves(pkg, dev):
+    """The layer seam's attention over the engine's pool, over a strided view
+    of a wider one and over a (K, V) pair of tensors: the same bits."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(0)
+    wide = torch.randn(3, 9, 16, 6, 128, generator=gen, device=dev).to(torch.bfloat16)
+    pool = wide[:2, 1:, :, 1:5]
+    q = torch.randn(3, 8, 128, generator=gen, device=dev).to(torch.bfloat16)
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=dev)  # noqa: E731
+    table = i32([[0, 3], [5, 1], [7, -1]])
+    metas = (pkg.DecodeAttentionMetadata(i32([20, 3, 9]), i32([0, 0, 0]), table, i32([21, 30, 10])),
+             pkg.PrefillAttentionMetadata(i32([18, 19, 5]), i32([0, 0, 0]), table, i32([0, 2, 3, 3]), i32([0, 20, 26, 26]),
+                                          None, None, 16))
+    for meta in metas:
+        outs = [pkg.attention_stored(kv, q, meta) for kv in (pool, pool.contiguous(), (pool[0], pool[1]))]
+        assert torch.isfinite(outs[0]).all() and outs[0][0].any()
+        assert all(torch.equal(o.view(torch.int16), outs[0].view(torch.int16)) for o in outs)
+    with pytest.raises(IndexError):
+        pkg.attention_stored(pool[:1], q, metas[0])

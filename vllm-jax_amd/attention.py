@@ -28,10 +28,10 @@ from typing import Optional, Tuple, Union
 import torch
 
 from . import _lib
-from .kernels._common import bf16_round, require_bf16, require_device, stream_handle
-from .kernels.decode_paged_attention import decode_paged_attention
+from .kernels._common import bf16_round, pool_pointers, require_bf16, require_device, stream_handle
+from .kernels.decode_paged_attention import decode_paged_attention, decode_pool
 from .kernels.mixed_paged_attention import mixed_paged_attention
-from .kernels.prefill_paged_attention import prefill_paged_attention
+from .kernels.prefill_paged_attention import prefill_paged_attention, prefill_pool
 
 USE_DECODE_PAGED_ATTENTION_KERNEL = True
 USE_PREFILL_PAGED_ATTENTION_KERNEL = True
@@ -129,15 +129,15 @@ def update_kv_cache(kv_cache: torch.Tensor, slot_mapping: torch.Tensor, k: torch
         raise ValueError("slot_mapping must be int32 of shape [T]")
     if _checking_slots():
         check_slot_mapping(slot_mapping, nb * bs)
-    kc, vc = kv_cache[0], kv_cache[1]
+    kc, vc = pool_pointers(kv_cache)
     sm = slot_mapping if slot_mapping.is_contiguous() else slot_mapping.contiguous()
     _lib.call(
         "pa_kv_store",
         k.data_ptr(), k.stride(0), k.stride(1),
         v.data_ptr(), v.stride(0), v.stride(1),
         sm.data_ptr(), k.shape[0], hkv, d,
-        kc.data_ptr(), vc.data_ptr(), nb, bs,
-        kc.stride(0), kc.stride(1), kc.stride(2),
+        kc, vc, nb, bs,
+        kv_cache.stride(1), kv_cache.stride(2), kv_cache.stride(3),
         stream_handle(k))
     return kv_cache
 
@@ -185,7 +185,7 @@ def qk_norm_rope_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm
         check_slot_mapping(slot_mapping, nb * bs)
     if out is None:
         out = torch.empty_like(q)
-    kc, vc = kv_cache[0], kv_cache[1]
+    kc, vc = pool_pointers(kv_cache)
     pos = positions.contiguous()
     sm = slot_mapping.contiguous()
     qw, kw = q_norm_weight.contiguous(), k_norm_weight.contiguous()
@@ -197,7 +197,7 @@ def qk_norm_rope_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm
         qw.data_ptr(), kw.data_ptr(), float(eps), float(rope_theta), factor,
         pos.data_ptr(), sm.data_ptr(), t_count, h, hkv, d,
         out.data_ptr(), out.stride(0), out.stride(1),
-        kc.data_ptr(), vc.data_ptr(), nb, bs, kc.stride(0), kc.stride(1), kc.stride(2),
+        kc, vc, nb, bs, kv_cache.stride(1), kv_cache.stride(2), kv_cache.stride(3),
         stream_handle(q))
     return out, kv_cache
 
@@ -229,12 +229,13 @@ def update_kv_cache_fp8(kv_codes: torch.Tensor, kv_scales: torch.Tensor, slot_ma
         raise ValueError("slot_mapping must be int32 of shape [T]")
     if _checking_slots():
         check_slot_mapping(slot_mapping, nb * bs)
-    kc, vc = kv_codes[0], kv_codes[1]
-    ks, vs = kv_scales[0], kv_scales[1]
+    kc, vc = pool_pointers(kv_codes)
+    ks, vs = pool_pointers(kv_scales)
     sm = slot_mapping.contiguous()
     _lib.call("pa_kv_store_fp8", k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(), v.stride(0), v.stride(1),
-              sm.data_ptr(), t_count, hkv, d, kc.data_ptr(), vc.data_ptr(), ks.data_ptr(), vs.data_ptr(),
-              nb, bs, kc.stride(0), kc.stride(1), kc.stride(2), ks.stride(1), ks.stride(2), ks.stride(0),
+              sm.data_ptr(), t_count, hkv, d, kc, vc, ks, vs,
+              nb, bs, kv_codes.stride(1), kv_codes.stride(2), kv_codes.stride(3),
+              kv_scales.stride(2), kv_scales.stride(3), kv_scales.stride(1),
               stream_handle(k))
     return kv_codes, kv_scales
 
@@ -264,25 +265,33 @@ def attention_stored(kv_cache: torch.Tensor, q: torch.Tensor, metadata: Attentio
     """The attention part of qwen3.py:175-218 for K/V already in the pool."""
     if not (USE_PREFILL_PAGED_ATTENTION_KERNEL and USE_DECODE_PAGED_ATTENTION_KERNEL):
         raise NotImplementedError("the dense fallbacks of qwen3.py:120-169 are not part of this library")
-    k_pages = kv_cache[0].permute(2, 0, 1, 3)   # [Hkv, NB, BS, d] view
-    v_pages = kv_cache[1].permute(2, 0, 1, 3)
+    head_dim = q.shape[-1]
+    # the engine's pool goes in as it is; anything else that has a K and a V
+    # half goes in as page views
+    pool = isinstance(kv_cache, torch.Tensor) and kv_cache.dim() == 5 and kv_cache.shape[0] >= 2
+    if isinstance(metadata, MixedAttentionMetadata) or not pool:
+        k_pages = kv_cache[0].permute(2, 0, 1, 3)   # [Hkv, NB, BS, d] view
+        v_pages = kv_cache[1].permute(2, 0, 1, 3)
     if isinstance(metadata, MixedAttentionMetadata):
-        head_dim = q.shape[-1]
         outputs = mixed_paged_attention(
             q, k_pages, v_pages, metadata.block_tables, metadata.cu_seqlens_q, metadata.kv_lens,
             metadata.input_positions, metadata.num_decodes, max_seqlen_q=metadata.max_seqlen_q,
             decode_scale=1.0 / bf16_round(float(head_dim) ** 0.5))
     elif isinstance(metadata, PrefillAttentionMetadata):
-        outputs = prefill_paged_attention(
-            q, k_pages, v_pages, metadata.block_tables, metadata.cu_seqlens_q,
-            metadata.slot_mapping, metadata.input_positions,
-            max_seqlen_bucket=metadata.max_seqlen_bucket,
-            cu_seqlens_k=metadata.cu_seqlens_k)
+        tables = (metadata.block_tables, metadata.cu_seqlens_q)
+        kw = dict(max_seqlen_bucket=metadata.max_seqlen_bucket, cu_seqlens_k=metadata.cu_seqlens_k)
+        if pool:
+            outputs = prefill_pool(q, kv_cache, *tables, metadata.input_positions, **kw)
+        else:
+            outputs = prefill_paged_attention(q, k_pages, v_pages, *tables, metadata.slot_mapping,
+                                              metadata.input_positions, **kw)
     else:
-        head_dim = q.shape[-1]
-        outputs = decode_paged_attention(
-            q, k_pages, v_pages, metadata.block_tables, metadata.context_lens,
-            scale=1.0 / bf16_round(float(head_dim) ** 0.5))
+        scale = 1.0 / bf16_round(float(head_dim) ** 0.5)
+        if pool:
+            outputs = decode_pool(q, kv_cache, metadata.block_tables, metadata.context_lens, scale=scale)
+        else:
+            outputs = decode_paged_attention(q, k_pages, v_pages, metadata.block_tables, metadata.context_lens,
+                                             scale=scale)
     return outputs
 
 

@@ -215,6 +215,31 @@ static float host_round_bf16(float x) {
   return r;
 }
 
+// inv_freq = 1 / theta ** (arange(0, d, 2) / d) with bf16 operands and results
+// (qwen3.py:62-63): theta, the exponent, the power and the reciprocal are each
+// rounded to bf16.  A model calls with one theta: each thread keeps the last
+// one's table (64 powers, 1.3 us of every call otherwise).
+static void rope_inv_freq(float rope_theta, uint32_t (&out)[kRopePairs / 2]) {
+  thread_local float kept = 0.f;  // never a valid theta
+  thread_local uint32_t table[kRopePairs / 2];
+  if (kept != rope_theta) {
+    const float theta = host_round_bf16(rope_theta);
+    for (int i = 0; i < kRopePairs / 2; ++i) {
+      uint32_t w = 0;
+      for (int h = 0; h < 2; ++h) {
+        const float e = host_round_bf16((float)(2 * (2 * i + h)) / (float)kRopeDim);
+        const float inv = host_round_bf16(1.f / host_round_bf16(powf(theta, e)));
+        uint32_t u;
+        memcpy(&u, &inv, 4);
+        w |= (u >> 16) << (16 * h);
+      }
+      table[i] = w;
+    }
+    kept = rope_theta;
+  }
+  memcpy(out, table, sizeof(table));
+}
+
 }  // namespace pa
 
 using namespace pa;
@@ -283,22 +308,7 @@ extern "C" int pa_qk_norm_rope_store(const uint16_t* q, int64_t q_tok_stride, in
   prm.eps = eps;
   prm.scale_pos = rope_scaling_factor != 1.f;
   prm.pos_div = rope_scaling_factor;
-  // inv_freq = 1 / theta ** (arange(0, d, 2) / d) with bf16 operands and
-  // results (qwen3.py:62-63): theta, the exponent, the power and the
-  // reciprocal are each rounded to bf16.
-  const float theta = host_round_bf16(rope_theta);
-  for (int i = 0; i < kRopePairs / 2; ++i) {
-    uint32_t w = 0;
-    for (int h = 0; h < 2; ++h) {
-      const float e = host_round_bf16((float)(2 * (2 * i + h)) / (float)head_dim);
-      const float pw = host_round_bf16(powf(theta, e));
-      const float inv = host_round_bf16(1.f / pw);
-      uint32_t u;
-      memcpy(&u, &inv, 4);
-      w |= (u >> 16) << (16 * h);
-    }
-    prm.inv_freq[i] = w;
-  }
+  rope_inv_freq(rope_theta, prm.inv_freq);
   prm.part_bits = rope_part_bits(num_tokens, (int64_t)num_heads + 2 * (int64_t)num_kv_heads);
   const int64_t blocks = (((int64_t)num_tokens << prm.part_bits) + 3) / 4;
   if (num_heads + 2 * num_kv_heads >= 64)

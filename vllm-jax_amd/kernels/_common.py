@@ -1,6 +1,7 @@
 """Shared argument plumbing for the kernel entry points (torch tensors -> C ABI)."""
 from __future__ import annotations
 
+import functools
 import math
 
 import numpy as np
@@ -10,6 +11,7 @@ import torch
 DEFAULT_MASK_VALUE = -0.7 * float(np.finfo(np.dtype("float32")).max)
 
 
+@functools.lru_cache(maxsize=64)  # of plain floats (a head size's scale, on every call); 10 us to evaluate
 def bf16_round(x: float) -> float:
     """The value a Python float takes when JAX weak-types it into bf16."""
     return float(torch.tensor(x, dtype=torch.float32).to(torch.bfloat16).float())
@@ -21,11 +23,12 @@ def inv_sqrt_head_dim_bf16(head_dim: int) -> float:
 
 
 def require_device(name: str, t: torch.Tensor) -> None:
+    if isinstance(t, torch.Tensor) and t.is_cuda:
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor, got {type(t).__name__}")
-    if t.device.type != "cuda":
-        raise ValueError(f"{name} must live on a HIP device (got {t.device}); "
-                         "the paged-attention path has no CPU implementation")
+    raise ValueError(f"{name} must live on a HIP device (got {t.device}); "
+                     "the paged-attention path has no CPU implementation")
 
 
 def require_bf16(name: str, t: torch.Tensor) -> None:
@@ -43,7 +46,14 @@ def as_i32(name: str, t: torch.Tensor) -> torch.Tensor:
 
 
 def stream_handle(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the handle alone: current_stream() builds a Stream object around it first
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+def pool_pointers(pool: torch.Tensor):
+    """Addresses of ``pool[0]`` and ``pool[1]`` (K and V), without making the views."""
+    k = pool.data_ptr()
+    return k, k + pool.stride(0) * pool.element_size()
 
 
 def pages_strides(k_pages: torch.Tensor):

@@ -20,7 +20,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from ._common import (DEFAULT_MASK_VALUE, as_i32, check_quantized_pages, pages_strides, require_bf16,
+from ._common import (DEFAULT_MASK_VALUE, as_i32, check_quantized_pages, pages_strides, pool_pointers, require_bf16,
                       require_device, stream_handle)
 
 
@@ -53,14 +53,45 @@ def decode_paged_attention(
 ) -> torch.Tensor:
     """Paged decode attention; q ``[B, H, d]`` -> ``[B, H, d]`` bf16."""
     del pages_per_compute_block, k_splits, num_warps, num_stages, interpret, debug, mask_value
-    batch_size, num_heads, head_dim = q.shape
-    num_kv_heads, total_num_pages, page_size, head_dim_k = k_pages.shape
-    batch_size_paged_indices, pages_per_sequence = block_tables.shape
-
     if tuple(k_pages.shape) != tuple(v_pages.shape):
         raise ValueError(
             f"k_pages and v_pages must have the same shape. Got {tuple(k_pages.shape)} and"
             f" {tuple(v_pages.shape)}")
+    _check_shapes(q, k_pages.shape, block_tables, lengths)
+    if block_h % 16:
+        raise ValueError(f"block_h must divisible by 16, but is {block_h}.")
+    code_type = check_quantized_pages(k_pages, v_pages, k_scales_pages, v_scales_pages)
+    for name, t in (("k_pages", k_pages), ("v_pages", v_pages)):
+        require_device(name, t)
+        if code_type is None:
+            require_bf16(name, t)
+    if tuple(k_pages.stride()) != tuple(v_pages.stride()):
+        raise ValueError("k_pages and v_pages must share strides")
+    num_kv_heads, num_pages, page_size, head_dim = k_pages.shape
+    scales = () if code_type is None else (k_scales_pages.data_ptr(), v_scales_pages.data_ptr(),
+                                           k_scales_pages.stride(1), k_scales_pages.stride(0))
+    return _decode(q, (num_kv_heads, num_pages, page_size, head_dim), (k_pages.data_ptr(), v_pages.data_ptr()),
+                   pages_strides(k_pages), code_type, scales, block_tables, lengths, attn_logits_soft_cap, scale,
+                   workspace, out)
+
+
+def decode_pool(q: torch.Tensor, kv_cache: torch.Tensor, block_tables: torch.Tensor, lengths: torch.Tensor | None,
+                *, scale: float) -> torch.Tensor:
+    """:func:`decode_paged_attention` over the halves of the engine's bf16
+    pool ``[2, NB, BS, Hkv, d]``, without making the page views."""
+    require_device("kv_cache", kv_cache)
+    require_bf16("kv_cache", kv_cache)
+    _, num_pages, page_size, num_kv_heads, head_dim = kv_cache.shape
+    _check_shapes(q, (num_kv_heads, num_pages, page_size, head_dim), block_tables, lengths)
+    _, ps, ss, hs, _ = kv_cache.stride()
+    return _decode(q, (num_kv_heads, num_pages, page_size, head_dim), pool_pointers(kv_cache), (ps, ss, hs), None, (),
+                   block_tables, lengths, None, scale, None, None)
+
+
+def _check_shapes(q, pages, block_tables, lengths):
+    batch_size, num_heads, head_dim = q.shape
+    num_kv_heads, head_dim_k = pages[0], pages[3]
+    batch_size_paged_indices = block_tables.shape[0]
     if num_heads % num_kv_heads != 0:
         raise ValueError(
             "Number of Q heads must be divisible by number of KV heads. Got"
@@ -76,21 +107,21 @@ def decode_paged_attention(
             raise ValueError("`lengths` and `q` must have the same batch size")
         if lengths.dtype != torch.int32:
             raise ValueError(f"The dtype of `lengths` must be int32. Got {lengths.dtype}")
-    if block_h % 16:
-        raise ValueError(f"block_h must divisible by 16, but is {block_h}.")
-    code_type = check_quantized_pages(k_pages, v_pages, k_scales_pages, v_scales_pages)
-    quantized = code_type is not None
 
-    for name, t in (("q", q), ("k_pages", k_pages), ("v_pages", v_pages), ("block_tables", block_tables)):
-        require_device(name, t)
+
+def _decode(q, pages, pointers, strides, code_type, scales, block_tables, lengths, attn_logits_soft_cap, scale,
+            workspace, out):
+    """The launch for checked pages: ``pages`` = (Hkv, NB, BS, d), ``pointers``
+    and element ``strides`` (page, slot, head) of K and V, ``scales`` =
+    pointers and (page, head) strides of quantized pages' scales."""
+    batch_size, num_heads, head_dim = q.shape
+    num_kv_heads, total_num_pages, page_size, _ = pages
+    pages_per_sequence = block_tables.shape[1]
+    require_device("q", q)
+    require_device("block_tables", block_tables)
     require_bf16("q", q)
-    if not quantized:
-        require_bf16("k_pages", k_pages)
-        require_bf16("v_pages", v_pages)
     if block_tables.dtype != torch.int32:
         raise ValueError("block_tables must be int32")
-    if tuple(k_pages.stride()) != tuple(v_pages.stride()):
-        raise ValueError("k_pages and v_pages must share strides")
     bt = block_tables if block_tables.stride(-1) == 1 else block_tables.contiguous()
     if lengths is None:
         lens = torch.full((batch_size,), pages_per_sequence * page_size, dtype=torch.int32, device=q.device)
@@ -108,14 +139,14 @@ def decode_paged_attention(
     if workspace is None or workspace.numel() * workspace.element_size() < need:
         workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
     soft_cap = 0.0 if attn_logits_soft_cap is None else float(attn_logits_soft_cap)
-    ps, ss, hs = pages_strides(k_pages)
-    if quantized:
+    ps, ss, hs = strides
+    if code_type is not None:
         _lib.call(
             "pa_decode_quant", code_type,
             q.data_ptr(), q.stride(0), q.stride(1),
-            k_pages.data_ptr(), v_pages.data_ptr(), k_scales_pages.data_ptr(), v_scales_pages.data_ptr(),
+            *pointers, scales[0], scales[1],
             total_num_pages, page_size, ps, ss, hs,
-            k_scales_pages.stride(1), k_scales_pages.stride(0),
+            scales[2], scales[3],
             bt.data_ptr(), bt.stride(0), pages_per_sequence,
             lens.data_ptr(), batch_size,
             num_heads, num_kv_heads, head_dim,
@@ -127,7 +158,7 @@ def decode_paged_attention(
     _lib.call(
         "pa_decode",
         q.data_ptr(), q.stride(0), q.stride(1),
-        k_pages.data_ptr(), v_pages.data_ptr(), total_num_pages, page_size,
+        *pointers, total_num_pages, page_size,
         ps, ss, hs,
         bt.data_ptr(), bt.stride(0), pages_per_sequence,
         lens.data_ptr(), batch_size,

@@ -20,7 +20,7 @@ import torch
 
 from .. import _lib
 from ._common import (DEFAULT_MASK_VALUE, as_i32, check_quantized_pages, inv_sqrt_head_dim_bf16, pages_strides,
-                      require_bf16, require_device, stream_handle)
+                      pool_pointers, require_bf16, require_device, stream_handle)
 
 
 def prefill_paged_attention(
@@ -70,13 +70,44 @@ def prefill_paged_attention(
     del interpret, debug, mask_value
     if block_h % 16:
         raise ValueError(f"block_h must divisible by 16, but is {block_h}.")
-    total_tokens, num_heads, head_dim = q.shape
-    num_kv_heads, total_num_pages, page_size, head_dim_k = k_pages.shape
-    batch, pages_per_sequence = block_tables.shape
     if tuple(k_pages.shape) != tuple(v_pages.shape):
         raise ValueError(
             f"k_pages and v_pages must have the same shape. Got {tuple(k_pages.shape)} and"
             f" {tuple(v_pages.shape)}")
+    _check_shapes(q, k_pages.shape, block_tables, cu_seqlens, cu_seqlens_k)
+    code_type = check_quantized_pages(k_pages, v_pages, k_scales_pages, v_scales_pages)
+    for name, t in (("k_pages", k_pages), ("v_pages", v_pages)):
+        require_device(name, t)
+        if code_type is None:
+            require_bf16(name, t)
+    if tuple(k_pages.stride()) != tuple(v_pages.stride()):
+        raise ValueError("k_pages and v_pages must share strides")
+    num_kv_heads, num_pages, page_size, head_dim = k_pages.shape
+    scales = () if code_type is None else (k_scales_pages.data_ptr(), v_scales_pages.data_ptr(),
+                                           k_scales_pages.stride(1), k_scales_pages.stride(0))
+    return _prefill(q, (num_kv_heads, num_pages, page_size, head_dim), (k_pages.data_ptr(), v_pages.data_ptr()),
+                    pages_strides(k_pages), code_type, scales, block_tables, cu_seqlens, input_positions,
+                    max_seqlen_bucket, attn_logits_soft_cap, cu_seqlens_k, scale, out, workspace)
+
+
+def prefill_pool(q: torch.Tensor, kv_cache: torch.Tensor, block_tables: torch.Tensor, cu_seqlens: torch.Tensor,
+                 input_positions: torch.Tensor, *, max_seqlen_bucket: int,
+                 cu_seqlens_k: torch.Tensor | None = None) -> torch.Tensor:
+    """:func:`prefill_paged_attention` over the halves of the engine's bf16
+    pool ``[2, NB, BS, Hkv, d]``, without making the page views."""
+    require_device("kv_cache", kv_cache)
+    require_bf16("kv_cache", kv_cache)
+    _, num_pages, page_size, num_kv_heads, head_dim = kv_cache.shape
+    _check_shapes(q, (num_kv_heads, num_pages, page_size, head_dim), block_tables, cu_seqlens, cu_seqlens_k)
+    _, ps, ss, hs, _ = kv_cache.stride()
+    return _prefill(q, (num_kv_heads, num_pages, page_size, head_dim), pool_pointers(kv_cache), (ps, ss, hs), None, (),
+                    block_tables, cu_seqlens, input_positions, max_seqlen_bucket, None, cu_seqlens_k, None, None, None)
+
+
+def _check_shapes(q, pages, block_tables, cu_seqlens, cu_seqlens_k):
+    num_heads, head_dim = q.shape[1:]
+    num_kv_heads, head_dim_k = pages[0], pages[3]
+    batch = block_tables.shape[0]
     if num_heads % num_kv_heads != 0:
         raise ValueError(
             "Number of Q heads must be divisible by number of KV heads. Got"
@@ -92,17 +123,19 @@ def prefill_paged_attention(
     if cu_seqlens_k is not None and tuple(cu_seqlens_k.shape) != (batch + 1,):
         raise ValueError("cu_seqlens_k must have shape [batch + 1]")
 
-    code_type = check_quantized_pages(k_pages, v_pages, k_scales_pages, v_scales_pages)
-    quantized = code_type is not None
-    for name, t in (("q", q), ("k_pages", k_pages), ("v_pages", v_pages), ("block_tables", block_tables),
-                    ("cu_seqlens", cu_seqlens), ("input_positions", input_positions)):
+
+def _prefill(q, pages, pointers, strides, code_type, scales, block_tables, cu_seqlens, input_positions,
+             max_seqlen_bucket, attn_logits_soft_cap, cu_seqlens_k, scale, out, workspace):
+    """The launch for checked pages: ``pages`` = (Hkv, NB, BS, d), ``pointers``
+    and element ``strides`` (page, slot, head) of K and V, ``scales`` =
+    pointers and (page, head) strides of quantized pages' scales."""
+    total_tokens, num_heads, head_dim = q.shape
+    num_kv_heads, total_num_pages, page_size, _ = pages
+    batch, pages_per_sequence = block_tables.shape
+    for name, t in (("q", q), ("block_tables", block_tables), ("cu_seqlens", cu_seqlens),
+                    ("input_positions", input_positions)):
         require_device(name, t)
     require_bf16("q", q)
-    if not quantized:
-        require_bf16("k_pages", k_pages)
-        require_bf16("v_pages", v_pages)
-    if tuple(k_pages.stride()) != tuple(v_pages.stride()):
-        raise ValueError("k_pages and v_pages must share strides")
     bt = block_tables if block_tables.stride(-1) == 1 else block_tables.contiguous()
     cu = as_i32("cu_seqlens", cu_seqlens)
     cuk = as_i32("cu_seqlens_k", cu_seqlens_k) if cu_seqlens_k is not None else None
@@ -117,7 +150,8 @@ def prefill_paged_attention(
     if scale is None:
         scale = inv_sqrt_head_dim_bf16(head_dim)
     soft_cap = 0.0 if attn_logits_soft_cap is None else float(attn_logits_soft_cap)
-    ps, ss, hs = pages_strides(k_pages)
+    ps, ss, hs = strides
+    quantized = code_type is not None
     lib = _lib.load()
     need = int(lib.pa_prefill_workspace_size(batch, int(max_seqlen_bucket), num_heads, num_kv_heads))
     extra = 0  # bytes of the widened pages
@@ -134,9 +168,9 @@ def prefill_paged_attention(
         _lib.call(
             "pa_prefill_quant", code_type,
             q.data_ptr(), q.stride(0), q.stride(1),
-            k_pages.data_ptr(), v_pages.data_ptr(), k_scales_pages.data_ptr(), v_scales_pages.data_ptr(),
+            *pointers, scales[0], scales[1],
             total_num_pages, page_size, ps, ss, hs,
-            k_scales_pages.stride(1), k_scales_pages.stride(0),
+            scales[2], scales[3],
             bt.data_ptr(), bt.stride(0), pages_per_sequence,
             cu.data_ptr(), cuk.data_ptr() if cuk is not None else None, pos.data_ptr(),
             batch, total_tokens, int(max_seqlen_bucket),
@@ -149,7 +183,7 @@ def prefill_paged_attention(
     _lib.call(
         "pa_prefill",
         q.data_ptr(), q.stride(0), q.stride(1),
-        k_pages.data_ptr(), v_pages.data_ptr(), total_num_pages, page_size,
+        *pointers, total_num_pages, page_size,
         ps, ss, hs,
         bt.data_ptr(), bt.stride(0), pages_per_sequence,
         cu.data_ptr(), cuk.data_ptr() if cuk is not None else None, pos.data_ptr(),
