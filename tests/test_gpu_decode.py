@@ -198,3 +198,22 @@ def test_decode_work_list_many_q_heads_per_kv_head(pkg, dev):
     print(f"decode G=64: {db.batch} sequences, table width {width}", flush=True)
     out, _ = _run_and_check(pkg, dev, db, seed=57)
     assert not u16(out)[0].any()
+
+
+@pytest.mark.parametrize("lens,h,hkv,bs,width", [
+    ([3000, 1, 0, 17, 2048, 511, 512, 513, 1025, 5000], 32, 8, 64, 128),    # ragged, empty sequences
+    ([1100] * 30 + [5] * 40, 32, 8, 256, 8),           # more parts than partial slots: parts of the cap
+    ([700, 4000, 33, 129], 16, 1, 32, 128),            # one kv head: a sequence in many parts, 32-token pages
+    ([900, 64, 2100, 1], 8, 8, 48, 64),                # 48-token pages
+    ([1024, 1023, 3000], 32, 8, 16, 256),              # 16-token pages: parts of up to 1024 tokens
+    ([600, 2300], 32, 8, 24, 128),                     # pages that are not whole steps
+    (list(range(1, 256)) + [480], 8, 4, 16, 32),       # 256 sequences, several rounds of single parts
+    ([2048 * 3], 24, 2, 64, 96),                       # G = 12
+])
+def test_decode_parts_cut_on_the_device(pkg, dev, lens, h, hkv, bs, width):
+    """Launches without a work list cut ragged sequences into equal parts by
+    an even share of the batch's tokens: every sequence against the oracle."""
+    db = wl.make_decode(lens, num_heads=h, num_kv_heads=hkv, page_size=bs, rng=np.random.default_rng(len(lens)),
+                        table_width=width)
+    out, _ = _run_and_check(pkg, dev, db, seed=5)
+    assert not ora.bf16_to_f32(u16(out))[np.asarray(lens) == 0].any()

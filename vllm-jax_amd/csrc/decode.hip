@@ -1,6 +1,7 @@
 // Split-K paged GQA decode for gfx950: the kernel entries and the host
 // launcher.  The work item (one chunk of one sequence and kv head) is
 // decode_item in decode_impl.h.
+#include <algorithm>
 #include <mutex>
 
 #include "any_head.h"
@@ -53,11 +54,143 @@ decode_plan_kernel(DecodeParams p, int32_t* __restrict__ plan) {
   if (tid == 0) plan[0] = count;
 }
 
+constexpr int kBalanceSlots = 512;    // workgroups resident at once (two per CU)
+constexpr int kBalanceMaxBatch = 256;  // one thread per sequence
+constexpr int kDecodeMinChunk = 512;   // shortest item of a small launch
+
+// Boundaries of a sequence's parts are multiples of this: whole steps, and of
+// 32-token pages whole pages (a 2048-token part then spans 64 of them).
+__host__ __device__ inline int balance_align(int page_size) { return page_size == 32 ? 32 : 16; }
+
+// Inclusive prefix sum over the wave's lanes: shifts inside the rows of 16
+// lanes, then the row totals broadcast to the rows above (DPP; the LDS
+// permutes of __shfl_up cost ten times the latency on this serial path).
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ uint32_t scan_dpp(uint32_t x) {
+  return x + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, kRowMask, 0xF, false);
+}
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
+  x = scan_dpp<0x111, 0xF>(x);  // row_shr:1
+  x = scan_dpp<0x112, 0xF>(x);  // row_shr:2
+  x = scan_dpp<0x114, 0xF>(x);  // row_shr:4
+  x = scan_dpp<0x118, 0xF>(x);  // row_shr:8
+  x = scan_dpp<0x142, 0xA>(x);  // row_bcast:15 into rows 1 and 3
+  x = scan_dpp<0x143, 0xC>(x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
+// ceil(x / d) for 0 <= x < 2^23, 0 < d < 2^23: a float quotient, put right.
+__device__ __forceinline__ int ceil_div_small(int x, int d) {
+  int q = (int)((float)x * __builtin_amdgcn_rcpf((float)d));
+  q -= q * d > x ? 1 : 0;
+  q += (q + 1) * d <= x ? 1 : 0;
+  return q + (q * d < x ? 1 : 0);
+}
+
+// The work item of workgroup blockIdx.x in a launch that cuts its sequences
+// on the device: every workgroup sums the lengths (one thread per sequence),
+// takes an even share of a resident workgroup as the part length L (at least
+// kDecodeMinChunk, at most p.balance_cap tokens), cuts each sequence into
+// equal parts of at most L and ranks the parts, those longer than L / 2
+// first, so that a ragged batch neither waits for its longest chunk nor
+// starts one last.  If that takes more partials than the workspace holds, L
+// is the cap, whose parts it is sized for.  XCD x = bid % 8 takes ranks x,
+// x + 8, ..., all kv heads of a rank in a row (as with the work list).  False:
+// nothing to do.
+// Against fixed chunks of 2048 tokens (1024 over 16-token pages) in sequence
+// order, whole calls in one process, Qwen3-8B heads: 16 sequences of 500 to
+// 16000 tokens 144.3 -> 121 us, 48 of 200 to 4000 98.0 -> 84, 24 of 200 to
+// 8000 over 16-token pages 107 -> 85, 128 of 100 to 2000 110.7 -> 98.
+__device__ __forceinline__ bool decode_balance(const DecodeParams& p, DecodeWork& w) {
+  __shared__ uint32_t s_sum[kDecodeWaves], s_cls[kDecodeWaves], s_slots[kDecodeWaves];
+  __shared__ int32_t s_work[7];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int hkv = p.num_kv_heads;
+  const int vheads = hkv * p.hblocks;
+  const int k = blockIdx.x >> 3;
+  const int kr = k / vheads;
+  const int mine = 8 * kr + (blockIdx.x & 7);
+  w.vh = k - kr * vheads;
+  // launches without a work list span fewer than 2^23 tokens over all table rows
+  const int len = tid < p.batch ? max(0, min(p.lengths[tid], p.pages_per_seq * p.page_size)) : 0;
+  const uint32_t sum = wave_scan((uint32_t)len);
+  if (lane == 63) s_sum[wave] = sum;
+  if (tid == 0) s_work[0] = -1;
+  __syncthreads();
+  const uint32_t total = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+  const int align = balance_align(p.page_size);
+  const uint64_t share = ((uint64_t)total * (uint32_t)vheads + kBalanceSlots - 1) / kBalanceSlots;
+  int most = share >= (uint64_t)p.balance_cap
+                 ? p.balance_cap
+                 : min(p.balance_cap, max(kDecodeMinChunk, ((int)share + align - 1) & -align));
+  int parts, size, start, slot;
+  while (true) {
+    size = (ceil_div_small(len, max(1, ceil_div_small(len, most))) + align - 1) & -align;
+    parts = ceil_div_small(len, max(size, align));
+    // parts of long (low half) and short parts; fewer than 2^16 of either
+    const bool small = 2 * size <= most;
+    const uint32_t mine_cls = (uint32_t)parts << (small ? 16 : 0);
+    uint32_t run = wave_scan(mine_cls);
+    slot = (int)wave_scan(parts > 1 ? (uint32_t)parts : 0u);
+    if (lane == 63) {
+      s_cls[wave] = run;
+      s_slots[wave] = (uint32_t)slot;
+    }
+    __syncthreads();
+    uint32_t all = 0;
+    int slots = 0;
+#pragma unroll
+    for (int i = 0; i < kDecodeWaves; ++i) {
+      run += i < wave ? s_cls[i] : 0;
+      slot += i < wave ? (int)s_slots[i] : 0;
+      all += s_cls[i];
+      slots += (int)s_slots[i];
+    }
+    start = (small ? (int)(run >> 16) + (int)(all & 0xffff) : (int)(run & 0xffff)) - parts;
+    slot -= parts > 1 ? parts : 0;
+    if (slots <= p.balance_slots || most == p.balance_cap) break;  // uniform
+    most = p.balance_cap;
+    __syncthreads();
+  }
+  if (mine >= start && mine < start + parts) {
+    const int i = mine - start;
+    s_work[0] = tid;
+    s_work[1] = i * size;
+    s_work[2] = min(i * size + size, len);
+    s_work[3] = len;
+    s_work[4] = parts;
+    s_work[5] = slot;
+    s_work[6] = i;
+  }
+  if (blockIdx.x == 0 && tid < p.batch) p.balance[tid] = (int32_t)((uint32_t)slot << 16 | (uint32_t)parts);
+  __syncthreads();
+  auto work = [&](int i) { return __builtin_amdgcn_readfirstlane(s_work[i]); };
+  w.b = work(0);
+  if (w.b < 0) return false;
+  w.t_begin = work(1);
+  w.t_end = work(2);
+  w.len = work(3);
+  const int n = work(4);
+  w.single = n == 1;
+  // a sequence's partials: its parts within each kv head
+  w.part = (int64_t)work(5) * hkv + (int64_t)(w.vh / p.hblocks) * n + work(6);
+  return true;
+}
+
 template <bool kAligned, bool kSoftCap, bool kFp8 = false, bool kShared = false, int kCode = kCodeE4M3,
           int kIds = 1>
 __global__ void __launch_bounds__(256, 2)
 decode_split_kernel(DecodeParams p) {
   __shared__ DecodeLds red;
+  if constexpr (kIds == 1) {
+    if (p.balance) {
+      DecodeWork w;
+      if (decode_balance(p, w))  // uniform over the workgroup
+        decode_run<kDecodeWaves, kAligned, kSoftCap, kFp8, kShared, kCode, kIds>(p, w, &red.o[0][0][0], &red.m[0][0],
+                                                                                 &red.l[0][0]);
+      return;
+    }
+  }
   int item;
   if (p.plan) {
     // XCD x = bid % 8 takes ranks x, x + 8, x + 16, ... of the list, all
@@ -80,6 +213,18 @@ decode_split_kernel(DecodeParams p) {
                                                                             &red.m[0][0], &red.l[0][0]);
 }
 
+// Parts nc of sequence b, and the first of its partials for kv head kvh.
+__device__ __forceinline__ int64_t decode_parts(const DecodeParams& p, int b, int kvh, int& nc) {
+  if (p.balance) {
+    const uint32_t rec = (uint32_t)p.balance[b];
+    nc = (int)(rec & 0xffffu);
+    return (int64_t)(rec >> 16) * p.num_kv_heads + (int64_t)kvh * nc;
+  }
+  const int len = min(p.lengths[b], p.pages_per_seq * p.page_size);
+  nc = len > 0 ? min((len + p.chunk - 1) / p.chunk, p.n_chunks) : 0;
+  return ((int64_t)b * p.num_kv_heads + kvh) * p.n_chunks;
+}
+
 // One wave per (sequence, q head): out = sum_c o_c 2^(m_c - M) / sum_c l_c 2^(m_c - M).
 // Sequences of one chunk were finished by the split kernel; length 0 gives zeros.
 __global__ void __launch_bounds__(256)
@@ -92,20 +237,22 @@ decode_merge_kernel(DecodeParams p) {
   if (!decode_has_row(p, b)) return;
   const int kvh = h / p.group;
   const int qi = h - kvh * p.group;
-  const int len = min(p.lengths[b], p.pages_per_seq * p.page_size);
-  const int nc = len > 0 ? min((len + p.chunk - 1) / p.chunk, p.n_chunks) : 0;
+  int nc;
+  const int64_t base = decode_parts(p, b, kvh, nc);
   if (nc == 1) return;
-  const int64_t base = ((int64_t)b * p.num_kv_heads + kvh) * p.n_chunks;
-  float mmax = -INFINITY;
-  for (int c = 0; c < nc; ++c) mmax = fmaxf(mmax, p.ws_ml[2 * ((base + c) * p.group + qi)]);
-  float o0 = 0.f, o1 = 0.f, lsum = 0.f;
+  // the sums follow a running max, so that no load waits for another part's
+  float m_run = -INFINITY, o0 = 0.f, o1 = 0.f, lsum = 0.f;
+#pragma unroll 4
   for (int c = 0; c < nc; ++c) {
     const int64_t part = (base + c) * p.group + qi;
-    const float w = fast_exp2(p.ws_ml[2 * part] - mmax);
-    lsum += p.ws_ml[2 * part + 1] * w;
+    const float2 ml = *reinterpret_cast<const float2*>(p.ws_ml + 2 * part);
     const float2 o = *reinterpret_cast<const float2*>(p.ws_o + part * kHeadDim + 2 * lane);
-    o0 += o.x * w;
-    o1 += o.y * w;
+    const float m_new = fmaxf(m_run, ml.x);  // finite: every part holds a token
+    const float old = fast_exp2(m_run - m_new), w = fast_exp2(ml.x - m_new);
+    m_run = m_new;
+    lsum = lsum * old + ml.y * w;
+    o0 = o0 * old + o.x * w;
+    o1 = o1 * old + o.y * w;
   }
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
   uint32_t* dst = reinterpret_cast<uint32_t*>(p.out + decode_row(p, b) * p.out_bs + (int64_t)h * p.out_hs) + lane;
@@ -128,10 +275,9 @@ decode_merge_wide_kernel(DecodeParams p) {
   if (!decode_has_row(p, b)) return;  // uniform over the workgroup
   const int kvh = h / p.group;
   const int qi = h - kvh * p.group;
-  const int len = min(p.lengths[b], p.pages_per_seq * p.page_size);
-  const int nc = len > 0 ? min((len + p.chunk - 1) / p.chunk, p.n_chunks) : 0;
+  int nc;
+  const int64_t base = decode_parts(p, b, kvh, nc);
   if (nc == 1) return;
-  const int64_t base = ((int64_t)b * p.num_kv_heads + kvh) * p.n_chunks;
   auto ml = [&](int c) __attribute__((always_inline)) { return p.ws_ml + 2 * ((base + c) * p.group + qi); };
   // M = the largest chunk max; L = sum_c l_c 2^(m_c - M)
   float mx = -INFINITY;
@@ -194,7 +340,6 @@ constexpr int kDecodeShortChunk = 1024;  // tokens per item of the generic decod
 // -1.3 %, 112 -1.2 %; 64 +1.6 %, 160 +1.6 %, 192 +3.6 %, 224 +1.9 %.
 static bool decode_any_short_chunk(int head_dim) { return head_dim < 128 && head_dim != 64; }
 
-constexpr int kDecodeMinChunk = 512;        // shortest item of a small launch
 constexpr int64_t kDecodeFillPairs = 64;  // (sequence, chunk) pairs of a launch that fills the CUs
 
 // A small launch (fewer than kDecodeFillPairs pairs over the widest table
@@ -317,6 +462,18 @@ extern "C" size_t pa_decode_workspace_size(int32_t batch, int32_t num_heads, int
   const int n_chunks = decode_chunks(batch, pages_per_seq, page_size, head_dim);
   const size_t pairs8 = ((size_t)batch * n_chunks + 7) / 8 * 8;
   return decode_partials_bytes(batch, num_heads, head_dim, n_chunks) + (kDecodePlanHeader + pairs8) * sizeof(int32_t);
+}
+
+// Whether a launch of `p` (with `fits`: decode_split_kernel's, without a work
+// list, and with pages) cuts its sequences on the device: not one sequence
+// alone (its chunks are equal; the cut costs about 1 us), and not when every
+// sequence is one short part and all of them are resident at once, where
+// neither the cut nor the order matters.  The token bound is decode_balance's
+// (any launch without a work list meets it at 8 kv heads and more).
+static bool decode_balanced(const DecodeParams& p, bool fits, int span, int64_t vheads) {
+  const int64_t tokens = (int64_t)p.pages_per_seq * p.page_size;
+  return fits && span <= 64 && p.batch > 1 && p.batch <= kBalanceMaxBatch && tokens * p.batch < (1 << 23) &&
+         (tokens > kDecodeMinChunk || p.batch * vheads > kBalanceSlots);
 }
 
 // Shared argument checks and launch of pa_decode / pa_decode_fp8.  `prm`
@@ -444,12 +601,21 @@ static int decode_common(const char* name, DecodeParams& prm, bool fp8, const ui
   // The work list pays for its launch once the grid is several waves of
   // workgroups deep (two per CU, 256 CUs).
   const bool planned = pairs > 0 && pairs * vheads >= kDecodePlanMinItems;
-  const int64_t blocks = planned ? (pairs + 7) / 8 * 8 * vheads : pairs * vheads;
+  int64_t blocks = planned ? (pairs + 7) / 8 * 8 * vheads : pairs * vheads;
   if (blocks > 0x7fffffff)
     return fail(PA_ERR_UNSUPPORTED, "%s: grid of %lld workgroups too large", name, (long long)blocks);
+  int32_t* plan = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(workspace) +
+                                             decode_partials_bytes(batch, num_heads, head_dim, prm.n_chunks));
+  if (decode_balanced(prm, !any_d && pairs > 0 && !planned, span, vheads)) {
+    prm.balance = plan;  // one int per sequence, in the work list's place
+    prm.balance_slots = (int32_t)pairs;
+    prm.balance_cap = decode_chunk_tokens(page_size);
+    // parts of at least an even share, or of the cap (decode_balance)
+    const int64_t cap_parts =
+        (int64_t)batch * (((int64_t)pages_per_seq * page_size + prm.balance_cap - 1) / prm.balance_cap);
+    blocks = (std::max<int64_t>(kBalanceSlots / vheads + batch, cap_parts) + 7) / 8 * 8 * vheads;
+  }
   if (planned) {
-    int32_t* plan = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(workspace) +
-                                               decode_partials_bytes(batch, num_heads, head_dim, prm.n_chunks));
     decode_plan_kernel<<<dim3(1), dim3(kPlanThreads), 0, s>>>(prm, plan);
     int rc = launch_status(name);
     if (rc) return rc;

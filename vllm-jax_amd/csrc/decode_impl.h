@@ -100,6 +100,11 @@ struct DecodeParams {
   // pairs, plan[kDecodePlanHeader + r] = pair index b * n_chunks + c of rank
   // r, most tokens first.
   const int32_t* plan;
+  // Launches that cut their sequences on the device (decode_balance; null
+  // otherwise): per sequence its parts, in the low half, and its first partial
+  // slot; the slots the workspace holds, and the longest part.
+  int32_t* balance;
+  int32_t balance_slots, balance_cap;
 };
 constexpr int kDecodePlanHeader = 64;  // ints before the first entry (256 bytes)
 
@@ -164,7 +169,17 @@ __device__ __forceinline__ int xcd_grouped_item(int bid, int nb) {
 // (one VGPR) a chunk spans at most 64 pages.
 __host__ __device__ inline int decode_chunk_tokens(int page_size) { return page_size >= 32 ? 2048 : 1024; }
 
-// One decode work item (sequence, chunk, kv head) numbered `item`, run by
+// A decode work item: tokens [t_begin, t_end) of sequence b (t_begin and, up
+// to the length, t_end multiples of 16) for (kv head, block of 16 q heads)
+// vh.  `single`: it holds the whole sequence and writes the output; else its
+// partial goes to rows `part` * group on of the workspace.
+struct DecodeWork {
+  int b, vh, t_begin, t_end, len;
+  bool single;
+  int64_t part;
+};
+
+// One decode work item, run by
 // kWaves wavefronts (threads 0 .. 64*kWaves-1 of the workgroup).  red_o /
 // red_m / red_l are LDS arrays of [kWaves][16][d] and [kWaves][16] floats.
 // kAligned: page_size % 16 == 0, so a 16-token step never crosses a page and
@@ -177,8 +192,8 @@ __host__ __device__ inline int decode_chunk_tokens(int page_size) { return page_
 // the K/V bytes of the bf16 path.
 template <int kWaves, bool kAligned, bool kSoftCap, bool kFp8 = false, bool kShared = false, int kCode = kCodeE4M3,
           int kIds = 1>
-__device__ __forceinline__ void decode_item(const DecodeParams& p, int item, float* red_o, float* red_m,
-                                            float* red_l) {
+__device__ __forceinline__ void decode_run(const DecodeParams& p, const DecodeWork& w, float* red_o, float* red_m,
+                                           float* red_l) {
   static_assert(kIds == 1 || kIds == 4, "one or four page ids per lane");
   static_assert(kWaves == 4 || kWaves == 8, "the combine splits d over the waves");
   static_assert(!kFp8 || kAligned, "float8 pages need 16-token aligned steps");
@@ -187,33 +202,12 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, int item, flo
   constexpr int kDPerLane = kDPerWave / 4;      // ... each lane (4 lane groups)
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int hkv = p.num_kv_heads;
-  const int vheads = hkv * p.hblocks;  // (kv head, block of 16 q heads) pairs
-  const int vh = item % vheads;
-  const int rest = item / vheads;
-  const int kvh = vh / p.hblocks;
-  const int qc0 = 16 * (vh - kvh * p.hblocks);  // first q column (head within the group) of this item
+  const int b = w.b, t_begin = w.t_begin, t_end = w.t_end, len = w.len;
+  const int kvh = w.vh / p.hblocks;
+  const int qc0 = 16 * (w.vh - kvh * p.hblocks);  // first q column (head within the group) of this item
   const int g_end = min(p.group, qc0 + 16);
-  const int chunk = rest % p.n_chunks;
-  const int b = rest / p.n_chunks;
-  // lengths past the block table's span are clamped to it (no read beyond the table row)
-  const int len = min(p.lengths[b], p.pages_per_seq * p.page_size);
-  if (!decode_has_row(p, b)) return;  // uniform over the workgroup
-  const int t_begin = chunk * p.chunk;
-  if (t_begin >= len) {  // uniform over the workgroup
-    if (chunk == 0 && p.zero_empty) {
-      // length 0: the G output rows of this kv head are zero
-      const int64_t orow = decode_row(p, b) * p.out_bs;
-      for (int c = threadIdx.x; c < (g_end - qc0) * (kHeadDim / 8); c += 64 * kWaves)
-        st16(p.out + orow + (int64_t)(kvh * p.group + qc0 + c / (kHeadDim / 8)) * p.out_hs + 8 * (c % (kHeadDim / 8)),
-             u32x4{0, 0, 0, 0});
-    }
-    return;
-  }
-  const int t_end = min(t_begin + p.chunk, len);
   const int n_steps = (t_end - t_begin + kDecodeStep - 1) / kDecodeStep;
   const int my_steps = n_steps > wave ? (n_steps - wave + kWaves - 1) / kWaves : 0;
-  const int n_chunks_b = (len + p.chunk - 1) / p.chunk;
 
   const int n = lane & 15;  // q column of S/O; the d chunk of V loads; the token of K loads
   const int g = lane >> 4;  // 16-lane group
@@ -503,7 +497,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, int item, flo
     }
   }
   if (qc0 + n >= g_end) return;
-  if (n_chunks_b == 1) {
+  if (w.single) {
     const float inv = 1.f / ll;  // ll >= 1: the chunk holds a visible token
     uint16_t* dst = p.out + decode_row(p, b) * p.out_bs + (int64_t)(kvh * p.group + qc0 + n) * p.out_hs + d0;
     if constexpr (kDPerLane == 8) {
@@ -518,7 +512,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, int item, flo
       *reinterpret_cast<u32x2*>(dst) = w;
     }
   } else {
-    const int64_t part = (((int64_t)b * hkv + kvh) * p.n_chunks + chunk) * p.group + qc0 + n;
+    const int64_t part = w.part * p.group + qc0 + n;
     float* dst = p.ws_o + part * kHeadDim + d0;
 #pragma unroll
     for (int i4 = 0; i4 < kDPerLane / 4; ++i4)
@@ -528,6 +522,42 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, int item, flo
       p.ws_ml[2 * part + 1] = ll;
     }
   }
+}
+
+// The item numbered `item` of a launch with fixed chunks: (sequence, chunk,
+// kv head and block of q heads), the latter fastest.
+template <int kWaves, bool kAligned, bool kSoftCap, bool kFp8 = false, bool kShared = false, int kCode = kCodeE4M3,
+          int kIds = 1>
+__device__ __forceinline__ void decode_item(const DecodeParams& p, int item, float* red_o, float* red_m,
+                                            float* red_l) {
+  const int hkv = p.num_kv_heads;
+  const int vheads = hkv * p.hblocks;  // (kv head, block of 16 q heads) pairs
+  DecodeWork w;
+  w.vh = item % vheads;
+  const int rest = item / vheads;
+  const int chunk = rest % p.n_chunks;
+  w.b = rest / p.n_chunks;
+  // lengths past the block table's span are clamped to it (no read beyond the table row)
+  w.len = min(p.lengths[w.b], p.pages_per_seq * p.page_size);
+  if (!decode_has_row(p, w.b)) return;  // uniform over the workgroup
+  w.t_begin = chunk * p.chunk;
+  const int kvh = w.vh / p.hblocks;
+  if (w.t_begin >= w.len) {  // uniform over the workgroup
+    if (chunk == 0 && p.zero_empty) {
+      // length 0: the G output rows of this kv head are zero
+      const int qc0 = 16 * (w.vh - kvh * p.hblocks);
+      const int g_end = min(p.group, qc0 + 16);
+      const int64_t orow = decode_row(p, w.b) * p.out_bs;
+      for (int c = threadIdx.x; c < (g_end - qc0) * (kHeadDim / 8); c += 64 * kWaves)
+        st16(p.out + orow + (int64_t)(kvh * p.group + qc0 + c / (kHeadDim / 8)) * p.out_hs + 8 * (c % (kHeadDim / 8)),
+             u32x4{0, 0, 0, 0});
+    }
+    return;
+  }
+  w.t_end = min(w.t_begin + p.chunk, w.len);
+  w.single = w.len <= p.chunk;
+  w.part = ((int64_t)w.b * hkv + kvh) * p.n_chunks + chunk;
+  decode_run<kWaves, kAligned, kSoftCap, kFp8, kShared, kCode, kIds>(p, w, red_o, red_m, red_l);
 }
 
 // Host launch of decode_merge_kernel for the sequences of `p` (defined with
