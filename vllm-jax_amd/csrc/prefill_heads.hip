@@ -12,11 +12,15 @@
 // by the ~7 us an item spends outside its loop at these lengths.  80 gained
 // nothing (492 us against 478, its generic kernel also fits two workgroups a
 // CU) and stays generic, as do the sizes between.
+#include <algorithm>
+
 #include "any_head.h"
 #include "prefill_impl.h"
 
 namespace pa {
 namespace {
+
+constexpr int kCUs = 256;
 
 // Tile paging of a launch at head size D; kPageLane: not one of the forms
 // built here (pages of other sizes, or rows too far apart for 32-bit offsets).
@@ -52,6 +56,12 @@ int prefill_tiled_launch(const char* name, const PrefillParams& prm, int head_di
   p.tile_tokens = kRows / p.group;
   p.n_qtiles = (p.max_seqlen_q + p.tile_tokens - 1) / p.tile_tokens;
   if (p.batch == 0 || p.max_seqlen_q == 0) return kPrefillNotTiled;
+  // At 256 the generic kernel's items are half as long (128 rows): while they
+  // fit one round on the CUs it is faster (3 x 299 tokens, 32 / 8 heads, 29.1
+  // us against 31.7; 2 x 300 behind 4000 cached 203 against 260), from there
+  // on this one (4 x 511 tokens 47 us against 52, 8 x 512 64 against 96).
+  const int64_t live = std::min<int64_t>((int64_t)p.batch * p.n_qtiles, p.num_tokens / p.tile_tokens + p.batch);
+  if (head_dim == 256 && live * p.num_kv_heads < kCUs / 2) return kPrefillNotTiled;
   const bool cap = p.soft_cap > 0.f;
   switch (head_dim) {
     case 64: return cap ? launch<64, true>(name, p, s) : launch<64, false>(name, p, s);

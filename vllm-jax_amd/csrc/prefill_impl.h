@@ -1017,16 +1017,20 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p, int bid) {
   if (prefill_resolve(p, bid, w)) prefill_run<kSoftCap, kPaging, D>(p, w);
 }
 
-// Output rows the prefill items do not write, for 64 tokens t0 .. t0 + 63
-// (one wave): rows outside all sequences (before cu_q[0], from cu_q[batch]
-// on) and rows at offset >= max_seqlen_q inside their sequence (the
-// reference drops those too: its scatter only covers the first
-// max_seqlen_bucket rows, prefill...:384-388) are zeroed.  A lane checks one
-// token; the wave zeroes the rows it found, one after the other.
+// Output rows the prefill items do not write, for kThreads tokens from t0 on
+// (one workgroup): rows outside all sequences (before cu_q[0], from
+// cu_q[batch] on) and rows at offset >= max_seqlen_q inside their sequence
+// (the reference drops those too: its scatter only covers the first
+// max_seqlen_bucket rows, prefill...:384-388) are zeroed.  A thread checks one
+// token; the rows found are dealt to all waves (a mixed step's decode rows
+// come before its prefill rows: 72 of them at head size 256 kept one wave
+// busy for 10 us).
 template <int D>
 __device__ __forceinline__ void prefill_zero_rows(const PrefillParams& p, int64_t t0) {
+  __shared__ unsigned long long s_todo[kWaves];
   const int lane = threadIdx.x & 63;
-  const int64_t t = t0 + lane;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t t = t0 + threadIdx.x;
   const int32_t* cu_q = p.cu_q;
   const int batch = p.batch;
   bool zero = t < p.num_tokens;
@@ -1040,15 +1044,24 @@ __device__ __forceinline__ void prefill_zero_rows(const PrefillParams& p, int64_
     }
     zero = t - cu_q[lo] >= p.max_seqlen_q;
   }
-  uint64_t todo = __ballot(zero);
+  const uint64_t found = __ballot(zero);
+  if (lane == 0) s_todo[wave] = found;
+  __syncthreads();
   const int chunks = p.num_heads * (D / 8);
-  while (todo) {
-    const int k = __ffsll((unsigned long long)todo) - 1;
-    todo &= todo - 1;
-    uint16_t* row = p.out + (t0 + k) * p.o_ts;
-    for (int c = lane; c < chunks; c += 64) {
-      const int hh = c / (D / 8);
-      st16(row + hh * p.o_hs + (c - hh * (D / 8)) * 8, u32x4{0, 0, 0, 0});
+  int turn = 0;  // wave `turn` takes the next row
+  for (int i = 0; i < kWaves; ++i) {
+    uint64_t todo = s_todo[i];
+    while (todo) {
+      const int k = __ffsll((unsigned long long)todo) - 1;
+      todo &= todo - 1;
+      if (turn == wave) {
+        uint16_t* row = p.out + (t0 + 64 * i + k) * p.o_ts;
+        for (int c = lane; c < chunks; c += 64) {
+          const int hh = c / (D / 8);
+          st16(row + hh * p.o_hs + (c - hh * (D / 8)) * 8, u32x4{0, 0, 0, 0});
+        }
+      }
+      turn = turn + 1 == kWaves ? 0 : turn + 1;
     }
   }
 }
@@ -1061,7 +1074,7 @@ prefill_kernel(PrefillParams p) {
   if constexpr (kZero) {
     const int64_t items = (int64_t)p.n_qtiles * p.batch * p.num_kv_heads;
     if (blockIdx.x >= items) {  // uniform over the workgroup
-      prefill_zero_rows<D>(p, ((int64_t)blockIdx.x - items) * kThreads + 64 * (threadIdx.x >> 6));
+      prefill_zero_rows<D>(p, ((int64_t)blockIdx.x - items) * kThreads);
       return;
     }
   }

@@ -52,7 +52,7 @@ template <bool kSoftCap, int kPaging>
 __global__ void __launch_bounds__(kThreads, 1)
 prefill_split_kernel(PrefillParams p, int grid_parts) {
   if ((int)blockIdx.x >= grid_parts) {  // uniform over the workgroup
-    prefill_zero_rows<kPHeadDim>(p, ((int64_t)blockIdx.x - grid_parts) * kThreads + 64 * (threadIdx.x >> 6));
+    prefill_zero_rows<kPHeadDim>(p, ((int64_t)blockIdx.x - grid_parts) * kThreads);
     return;
   }
   __shared__ unsigned long long s_total;
