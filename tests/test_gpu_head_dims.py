@@ -61,6 +61,20 @@ def test_prefill_head_dims_tiled(pkg, dev, d, tile, bs, cap):
     _prefill(pkg, dev, pb, seed=d + bs, soft_cap=cap, use_seam=cap is None)
 
 
+@pytest.mark.parametrize("d,bs,cap", [(64, 64, None), (96, 16, None), (256, 32, 8.0)])
+def test_prefill_head_dims_tiled_work_list(pkg, dev, d, bs, cap):
+    """Launches large enough for the work list (70 sequences, 2 q tiles, 8 kv
+    heads: 1 120 items), padded rows among them, every sequence against the
+    oracle."""
+    rng = np.random.default_rng(d)
+    lens = rng.integers(1, 129, size=70)
+    lens[:4] = [128, 1, 64, 65]
+    pb = wl.make_prefill(lens, num_heads=32, num_kv_heads=8, page_size=bs, head_dim=d, rng=rng,
+                         pad_tokens_to=int(lens.sum()) + 37)
+    got, _ = _prefill(pkg, dev, pb, seed=d, soft_cap=cap, use_seam=cap is None)
+    assert not got[int(lens.sum()):].any()
+
+
 @pytest.mark.parametrize("d", [64, 96, 256])
 def test_prefill_head_dims_tiled_equals_generic(pkg, dev, d):
     """The same tokens over 32-token pages (tiled kernel) and over 24-token

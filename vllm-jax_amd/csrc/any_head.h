@@ -14,13 +14,18 @@ struct DecodeParams;
 bool any_head_dim(int head_dim);
 
 // Prefill of `p` with the tiled ping-pong kernel at the head sizes and page
-// sizes it is built for (prefill_heads.hip), rows no item covers zeroed;
-// kPrefillNotTiled, with nothing launched, for any other.  Else a PA_* code.
+// sizes it is built for (prefill_heads.hip); kPrefillNotTiled, with nothing
+// launched, for any other.  With the work list p.plan (items of 256 rows) the
+// rows no item covers are the caller's; without one they are zeroed here.
+// Else a PA_* code.
 constexpr int kPrefillNotTiled = 1;
 int prefill_tiled_launch(const char* name, const PrefillParams& p, int head_dim, hipStream_t s);
+// Whether prefill_tiled_launch takes `p`.
+bool prefill_tiled(const PrefillParams& p, int head_dim);
 
-// Zero pass and prefill of `p` (filled as for the tuned kernel; the work
-// list and pools are not used) with `head_dim`-wide rows.  Returns a PA_*
+// Prefill of `p` (filled as for the tuned kernel) with `head_dim`-wide rows:
+// the tiled kernel where it fits, else the zero pass and the generic kernel
+// (the work list and pools are not used).  Returns a PA_*
 // code.
 int prefill_any_launch(const char* name, const PrefillParams& p, int head_dim, hipStream_t s);
 

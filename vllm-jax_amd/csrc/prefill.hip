@@ -148,7 +148,7 @@ __device__ void prefill_plan(const PrefillParams& p, int32_t* __restrict__ plan)
 // too: its scatter only covers the first max_seqlen_bucket rows,
 // prefill...:384-388).  One wave per token row.
 __global__ void __launch_bounds__(kPrepThreads)
-prefill_prep_kernel(PrefillParams p, int32_t* __restrict__ plan) {
+prefill_prep_kernel(PrefillParams p, int32_t* __restrict__ plan, int head_dim) {
   int zb = blockIdx.x;
   if (plan) {
     if (zb == 0) {
@@ -174,7 +174,7 @@ prefill_prep_kernel(PrefillParams p, int32_t* __restrict__ plan) {
     covered = t - cu_q[lo] < p.max_seqlen_q;
   }
   if (covered) return;
-  const int chunks_per_head = kPHeadDim / 8;
+  const int chunks_per_head = head_dim / 8;
   for (int c = lane; c < p.num_heads * chunks_per_head; c += 64) {
     const int hh = c / chunks_per_head;
     const int e = (c - hh * chunks_per_head) * 8;
@@ -460,7 +460,10 @@ static int prefill_launch(const char* name, const uint16_t* q, int64_t q_tok_str
   prm.o_ts = out_tok_stride;
   prm.o_hs = out_head_stride;
 #ifndef PA_PREFILL_PHASES
-  if (any_d) return prefill_any_launch(name, prm, head_dim, s);
+  const bool tiled_d = any_d && prefill_tiled(prm, head_dim);
+  if (any_d && !tiled_d) return prefill_any_launch(name, prm, head_dim, s);
+#else
+  const bool tiled_d = false;
 #endif
   const int64_t items = (int64_t)prm.n_qtiles * batch * num_kv_heads;
   if (items > 0x7fffffff)
@@ -469,7 +472,7 @@ static int prefill_launch(const char* name, const uint16_t* q, int64_t q_tok_str
   const bool planned = workspace && batch > 0 && max_seqlen_q > 0 && batch <= kPlanMaxBatch &&
                        items >= kPrefillPlanMinItems;
 #ifndef PA_PREFILL_PHASES
-  if (workspace && !planned && batch > 0 && prefill_splits(prm)) {  // few items: split the long ones if the workspace holds their partials
+  if (!any_d && workspace && !planned && batch > 0 && prefill_splits(prm)) {  // few items: split the long ones if the workspace holds their partials
     const size_t split = prefill_split_bytes(batch, prm.n_qtiles, num_kv_heads, (int64_t)pages_per_seq * page_size);
     if (split && workspace_bytes >= split)
       return prefill_split_launch(name, prm, prefill_paging(page_size, slot_stride), workspace, s);
@@ -478,11 +481,14 @@ static int prefill_launch(const char* name, const uint16_t* q, int64_t q_tok_str
   int32_t* plan = planned ? reinterpret_cast<int32_t*>(workspace) : nullptr;
   if (planned) {  // the list and the zero rows, ahead of the prefill
     const int64_t zero_blocks = (num_tokens + kPrepThreads / 64 - 1) / (kPrepThreads / 64) + 1;
-    prefill_prep_kernel<<<dim3((unsigned)zero_blocks), dim3(kPrepThreads), 0, s>>>(prm, plan);
+    prefill_prep_kernel<<<dim3((unsigned)zero_blocks), dim3(kPrepThreads), 0, s>>>(prm, plan, head_dim);
     int rc = launch_status(name);
     if (rc) return rc;
   }
   prm.plan = plan;
+#ifndef PA_PREFILL_PHASES
+  if (tiled_d) return prefill_any_launch(name, prm, head_dim, s);
+#endif
   // the pool pays off on long launches (the XCDs' finishing spread grows with
   // the launch; the extra workgroups cost a dispatch each)
   prm.pool = plan && num_kv_heads % 8 == 0 && items >= kPoolMinItems ? plan + 8 : nullptr;

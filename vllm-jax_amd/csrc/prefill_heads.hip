@@ -13,6 +13,7 @@
 // nothing (492 us against 478, its generic kernel also fits two workgroups a
 // CU) and stays generic, as do the sizes between.
 #include <algorithm>
+#include <type_traits>
 
 #include "any_head.h"
 #include "prefill_impl.h"
@@ -36,32 +37,54 @@ int tiled_paging(int32_t page_size, int64_t slot_stride) {
 template <int D, bool kSoftCap>
 int launch(const char* name, const PrefillParams& p, hipStream_t s) {
   const int paging = tiled_paging<D, kSoftCap>(p.page_size, p.slot_stride);
-  if (paging == kPageLane) return kPrefillNotTiled;
   const int64_t items = (int64_t)p.n_qtiles * p.batch * p.num_kv_heads;
-  // workgroups past the items zero the rows no item writes, 512 tokens each
-  const int64_t blocks = items + ((int64_t)p.num_tokens + kThreads - 1) / kThreads;
-  if (blocks > 0x7fffffff) return kPrefillNotTiled;
+  // without a list, workgroups past the items zero the rows no item writes,
+  // 512 tokens each
+  const int64_t blocks = items + (p.plan ? 0 : ((int64_t)p.num_tokens + kThreads - 1) / kThreads);
+  if (blocks > 0x7fffffff)
+    return fail(PA_ERR_UNSUPPORTED, "%s: grid of %lld workgroups too large", name, (long long)blocks);
   const dim3 g((unsigned)blocks), b(kThreads);
-  if (paging == kPageTile) prefill_kernel<kSoftCap, kPageTile, true, D><<<g, b, 0, s>>>(p);
-  else prefill_kernel<kSoftCap, kPageWave, true, D><<<g, b, 0, s>>>(p);
+  auto run = [&](auto pg) {
+    constexpr int kPg = decltype(pg)::value;
+    if (p.plan) prefill_kernel<kSoftCap, kPg, false, D><<<g, b, 0, s>>>(p);
+    else prefill_kernel<kSoftCap, kPg, true, D><<<g, b, 0, s>>>(p);
+  };
+  if (paging == kPageTile) run(std::integral_constant<int, kPageTile>{});
+  else run(std::integral_constant<int, kPageWave>{});
   return launch_status(name);
+}
+
+template <int D>
+int paging_of(const PrefillParams& p) {
+  return p.soft_cap > 0.f ? tiled_paging<D, true>(p.page_size, p.slot_stride)
+                          : tiled_paging<D, false>(p.page_size, p.slot_stride);
 }
 
 }  // namespace
 
-int prefill_tiled_launch(const char* name, const PrefillParams& prm, int head_dim, hipStream_t s) {
-  PrefillParams p = prm;
-  p.plan = nullptr;
-  p.pool = nullptr;
-  p.tile_tokens = kRows / p.group;
-  p.n_qtiles = (p.max_seqlen_q + p.tile_tokens - 1) / p.tile_tokens;
-  if (p.batch == 0 || p.max_seqlen_q == 0) return kPrefillNotTiled;
+bool prefill_tiled(const PrefillParams& p, int head_dim) {
+  if (p.batch == 0 || p.max_seqlen_q == 0) return false;
+  const int64_t tile_tokens = kRows / p.group;
+  const int64_t pairs = p.batch * ((p.max_seqlen_q + tile_tokens - 1) / tile_tokens);
   // At 256 the generic kernel's items are half as long (128 rows): while they
   // fit one round on the CUs it is faster (3 x 299 tokens, 32 / 8 heads, 29.1
   // us against 31.7; 2 x 300 behind 4000 cached 203 against 260), from there
   // on this one (4 x 511 tokens 47 us against 52, 8 x 512 64 against 96).
-  const int64_t live = std::min<int64_t>((int64_t)p.batch * p.n_qtiles, p.num_tokens / p.tile_tokens + p.batch);
-  if (head_dim == 256 && live * p.num_kv_heads < kCUs / 2) return kPrefillNotTiled;
+  const int64_t live = std::min<int64_t>(pairs, p.num_tokens / tile_tokens + p.batch);
+  switch (head_dim) {
+    case 64: return paging_of<64>(p) != kPageLane;
+    case 96: return paging_of<96>(p) != kPageLane;
+    case 256: return p.group <= 128 && paging_of<256>(p) != kPageLane && live * p.num_kv_heads >= kCUs / 2;
+    default: return false;
+  }
+}
+
+int prefill_tiled_launch(const char* name, const PrefillParams& prm, int head_dim, hipStream_t s) {
+  if (!prefill_tiled(prm, head_dim)) return kPrefillNotTiled;
+  PrefillParams p = prm;
+  p.pool = nullptr;
+  p.tile_tokens = kRows / p.group;
+  p.n_qtiles = (p.max_seqlen_q + p.tile_tokens - 1) / p.tile_tokens;
   const bool cap = p.soft_cap > 0.f;
   switch (head_dim) {
     case 64: return cap ? launch<64, true>(name, p, s) : launch<64, false>(name, p, s);
