@@ -2,8 +2,9 @@
 // 256): a prefill kernel and a split-K decode kernel with its merge.  The
 // reference takes any head size as long as q and the pages agree
 // (prefill_paged_attention.py:199-203, decode_paged_attention.py:356-360);
-// the tuned kernels of prefill.hip / decode.hip are built for 128, and these
-// cover the rest with the same arithmetic: S in f32 on the matrix core from
+// the tuned kernels of prefill.hip / decode.hip are built for 128 (the
+// prefill also for 64, 96 and 256 over common page sizes, prefill_heads.hip),
+// and these cover the rest with the same arithmetic: S in f32 on the matrix core from
 // bf16 q (scaled by scale * log2 e and rounded, without the soft cap) and K,
 // exp2 online softmax with a lazily moved reference max, P rounded to bf16
 // for PV, f32 O.
