@@ -349,3 +349,45 @@ def test_prefill_split_workspace_size():
                  (0, 512, 32, 8, 128, 64, 256)):
         assert size(*args) == plan(*args[:4])
     assert size(2, 512, 33, 8, 128, 64, 256) == 0
+
+
+@pytest.mark.parametrize("tokens,cached,heads,hkv,tiled", [
+    # (new tokens, cached tokens) per sequence at head size 256, 256-token
+    # pages and exact tables; one round of generic items stays generic
+    ([299] * 3, 0, 32, 8, False), ([1000], 0, 32, 8, False), ([1000], 4000, 32, 8, False),
+    ([500] * 2, 4000, 32, 8, False), ([100] * 8, 4000, 32, 8, False), ([250] * 4, 0, 32, 8, False),
+    ([511] * 4, 0, 16, 8, False), ([1000] * 2, 4000, 16, 8, False), ([512] * 8, 0, 8, 8, False),
+    ([4000], 0, 8, 4, False), ([30] * 20, 0, 8, 8, False),
+    # more than a round, but the longest item decides
+    ([1500], 0, 32, 8, False), ([2000], 0, 32, 8, False), ([700] * 2, 0, 32, 8, False),
+    ([4000], 0, 16, 8, False), ([1400] * 2, 0, 16, 8, False), ([4000], 0, 16, 1, False),
+    # several rounds
+    ([3000], 0, 32, 8, True), ([511] * 4, 0, 32, 8, True), ([200] * 5, 0, 32, 8, True),
+    ([1000] * 2, 4000, 32, 8, True), ([300] * 4, 4000, 32, 8, True), ([128] * 16, 0, 32, 8, True),
+    ([1500], 0, 64, 8, True), ([2000] * 16, 0, 32, 8, True),
+    # half-filled tiles
+    ([64] * 8, 4000, 8, 8, True), ([32] * 32, 0, 32, 8, True),
+])
+def test_prefill_route_at_head_size_256(tokens, cached, heads, hkv, tiled):
+    """The kernel that was faster when both were timed (prefill_heads.hip)."""
+    route = PKG._lib.load().pa_prefill_route
+    pages = -(-(max(tokens) + cached) // 256)
+    bucket = 1 << (max(tokens) - 1).bit_length()
+    assert route(len(tokens), sum(tokens), bucket, heads, hkv, 256, pages, 256, 1) == tiled
+    # nothing cached, in a table for 32k tokens: as the exact table says
+    if not cached:
+        assert route(len(tokens), sum(tokens), max(tokens), heads, hkv, 256, 128, 256, 0) == tiled
+
+
+def test_prefill_route_edges():
+    route = PKG._lib.load().pa_prefill_route
+    assert route(1, 100, 100, 32, 8, 128, 1, 256, 1) == 1
+    assert route(1, 100, 100, 32, 8, 64, 1, 256, 1) == 1
+    assert route(1, 100, 100, 32, 8, 64, 10, 24, 1) == 0      # pages of another size
+    assert route(1, 100, 100, 32, 8, 80, 1, 256, 1) == 0      # head size not tiled
+    assert route(64, 1 << 16, 2048, 256, 1, 256, 8, 256, 1) == 0  # more than 128 q heads per kv head
+    for bad in ((-1, 100, 100, 32, 8, 128, 1, 256, 1), (1, 100, 100, 32, 7, 128, 1, 256, 1),
+                (1, 100, 100, 32, 8, 100, 1, 256, 1), (1, 100, 100, 32, 8, 128, 1, 0, 1)):
+        assert route(*bad) == -1
+    for empty in ((0, 0, 0), (0, 5, 0), (1, 0, 100), (1, 5, 0)):
+        assert route(*empty, 32, 8, 256, 0, 256, 1) in (0, 1)

@@ -56,8 +56,11 @@ def test_prefill_head_dims_tiled(pkg, dev, d, tile, bs, cap):
     four-iteration loop, groups whose last rows are idle, every sequence
     against the oracle."""
     lens = [1, tile - 1, tile, tile + 1, 4 * tile + 1, 5 * tile, 6 * tile - 1, 7 * tile + 2]
-    pb = wl.make_prefill(lens, num_heads=12, num_kv_heads=2, page_size=bs, head_dim=d,
+    hkv = 8 if d == 256 else 2  # 256 is tiled from several rounds of items on
+    pb = wl.make_prefill(lens, num_heads=6 * hkv, num_kv_heads=hkv, page_size=bs, head_dim=d,
                          rng=np.random.default_rng(bs + d))
+    assert pkg._lib.load().pa_prefill_route(len(lens), sum(lens), pb.max_seqlen_bucket, 6 * hkv, hkv, d,
+                                            pb.block_tables.shape[1], bs, 1) == 1
     _prefill(pkg, dev, pb, seed=d + bs, soft_cap=cap, use_seam=cap is None)
 
 
@@ -71,6 +74,8 @@ def test_prefill_head_dims_tiled_work_list(pkg, dev, d, bs, cap):
     lens[:4] = [128, 1, 64, 65]
     pb = wl.make_prefill(lens, num_heads=32, num_kv_heads=8, page_size=bs, head_dim=d, rng=rng,
                          pad_tokens_to=int(lens.sum()) + 37)
+    assert pkg._lib.load().pa_prefill_route(70, int(lens.sum()) + 37, pb.max_seqlen_bucket, 32, 8, d,
+                                            pb.block_tables.shape[1], bs, 1) == 1
     got, _ = _prefill(pkg, dev, pb, seed=d, soft_cap=cap, use_seam=cap is None)
     assert not got[int(lens.sum()):].any()
 
@@ -83,7 +88,7 @@ def test_prefill_head_dims_tiled_equals_generic(pkg, dev, d):
     (2^-9 relative each), O(1) values, so they differ by at most 2e-2."""
     import torch
     gen = torch.Generator(device=dev).manual_seed(d)
-    h, hkv = 8, 4
+    h, hkv = (64, 32) if d == 256 else (8, 4)  # 256 is tiled from several rounds of items on
     new, pre = [70, 1, 133, 300], [0, 500, 61, 127]
     cu = np.concatenate([[0], np.cumsum(new)])
     cu_k = np.concatenate([[0], np.cumsum(np.add(new, pre))])
@@ -98,6 +103,7 @@ def test_prefill_head_dims_tiled_equals_generic(pkg, dev, d):
         pages = [-(-int(n) // bs) for n in np.diff(cu_k)]
         nb = sum(pages) + 2
         table = np.full((len(new), max(pages)), -1, np.int32)
+        assert pkg._lib.load().pa_prefill_route(len(new), t, 256, h, hkv, d, max(pages), bs, 1) == (bs == 32)
         pool = torch.zeros((2, nb, bs, hkv, d), dtype=torch.bfloat16, device=dev)
         at = 0
         for b, n in enumerate(pages):

@@ -113,6 +113,7 @@ SIGNATURES = {
         c_vp, c_sz, c_vp,              # workspace, bytes, stream
     ]),
     "pa_prefill_split_workspace_size": (c_sz, [c_i32] * 7),
+    "pa_prefill_route": (ctypes.c_int, [c_i32] * 9),
     "pa_prefill_fp8_workspace_size": (c_sz, [c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32]),
     "pa_prefill_fp8": (ctypes.c_int, [
         c_vp, c_i64, c_i64,            # q

@@ -543,6 +543,33 @@ extern "C" size_t pa_prefill_split_workspace_size(int32_t batch, int32_t max_seq
 }
 #endif
 
+#ifndef PA_PREFILL_PHASES
+extern "C" int pa_prefill_route(int32_t batch, int32_t num_tokens, int32_t max_seqlen_q, int32_t num_heads,
+                                int32_t num_kv_heads, int32_t head_dim, int32_t pages_per_seq, int32_t page_size,
+                                int32_t cached) {
+  if (batch < 0 || num_tokens < 0 || max_seqlen_q < 0 || num_heads <= 0 || num_kv_heads <= 0 ||
+      num_heads % num_kv_heads || num_heads / num_kv_heads > kRows || pages_per_seq < 0 || page_size <= 0 ||
+      (head_dim != kPHeadDim && !any_head_dim(head_dim)))
+    return fail(PA_ERR_INVALID_ARGUMENT, "pa_prefill_route: bad sizes");
+  const int32_t cu = 0;  // never read: cu_k only says whether tokens are cached
+  PrefillParams p{};
+  p.cu_k = cached ? &cu : nullptr;
+  p.batch = batch;
+  p.num_tokens = num_tokens;
+  p.max_seqlen_q = max_seqlen_q;
+  p.num_heads = num_heads;
+  p.num_kv_heads = num_kv_heads;
+  p.group = num_heads / num_kv_heads;
+  p.pages_per_seq = pages_per_seq;
+  p.page_size = page_size;
+  p.slot_stride = (int64_t)num_kv_heads * head_dim;
+  p.tile_tokens = kRows / p.group;
+  p.n_qtiles = (max_seqlen_q + p.tile_tokens - 1) / p.tile_tokens;
+  if (head_dim != kPHeadDim) return prefill_tiled(p, head_dim) ? PA_PREFILL_TILED : PA_PREFILL_GENERIC;
+  return PA_PREFILL_TILED;
+}
+#endif
+
 extern "C" int pa_prefill(const uint16_t* q, int64_t q_tok_stride, int64_t q_head_stride,
                           const uint16_t* k_cache, const uint16_t* v_cache,
                           int32_t num_pages, int32_t page_size,

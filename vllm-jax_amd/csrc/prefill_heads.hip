@@ -13,6 +13,7 @@
 // nothing (492 us against 478, its generic kernel also fits two workgroups a
 // CU) and stays generic, as do the sizes between.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "any_head.h"
@@ -62,19 +63,56 @@ int paging_of(const PrefillParams& p) {
 
 }  // namespace
 
+// Items of `tokens`-token tiles a launch can have at most: a sequence of n
+// tokens has ceil(n / tokens) of them per kv head.
+static int64_t items_of(const PrefillParams& p, int64_t tokens) {
+  const int64_t grid = p.batch * ((p.max_seqlen_q + tokens - 1) / tokens);
+  return std::min(grid, (p.num_tokens + p.batch * (tokens - 1)) / tokens) * p.num_kv_heads;
+}
+
+// Whether a launch at head size 256 is faster tiled than in the generic
+// kernel.  The generic kernel's items are half as long (128 rows against 256)
+// and each is done sooner: 12 us and 44 ns a kv token on a CU of its own,
+// against 10 us and 57 ns.  So a launch whose generic items fit one round on
+// the CUs stays generic, unless its sequences fill at most half a tile, where
+// the tiled kernel's other waves skip their work; a launch of several rounds
+// is tiled, and in between the two estimates decide: the longest item, or all
+// of them over the CUs.  kv lengths are on the device.  The longest is taken
+// from the table's width, or, where cu_seqlens_k says that nothing is cached
+// (and in a mixed launch, whose table is as wide as its decode sequences),
+// from max_seqlen_q; the others are taken to be as long.
+// Generic -> tiled, 32 / 8 heads unless said, us (both kernels measured at 400
+// shapes; this rule takes the slower one by 4 % at most, in 4 of them): generic
+// 3 x 299 tokens 28.0 -> 31.5, 1 x 2000 118 -> 131, 1 x 1000 behind 4000
+// cached 237 -> 302, 16 / 8 heads 1 x 4000 211 -> 246; tiled 4 x 511 50.3 ->
+// 46.6, 1 x 3000 258 -> 190, 4 x 300 behind 4000 384 -> 265, 8 / 8 heads 8 x 64
+// behind 4000 223 -> 175.
+static bool tiled_256_pays(const PrefillParams& p) {
+  const int rows = 128;  // of a generic item
+  const double mean = (double)p.num_tokens / p.batch;
+  const double span = (double)p.pages_per_seq * p.page_size;
+  const int64_t seq_rows = (int64_t)p.max_seqlen_q * p.group;
+  if (seq_rows > 32 && seq_rows <= rows) return true;
+  if (seq_rows > 32 && seq_rows <= kRows && mean <= 64 && span <= 256) return true;
+  const int64_t generic = items_of(p, rows / p.group), tiled = items_of(p, kRows / p.group);
+  if (generic <= kCUs && (int64_t)p.num_tokens * p.num_heads < (int64_t)kCUs * rows) return false;
+  const bool fresh = p.kv_lens || !p.cu_k || p.cu_k == p.cu_q;
+  const double longest = fresh ? std::min<double>(span, p.max_seqlen_q) : std::max(span - p.page_size + 1, mean);
+  const double average = longest - std::min(mean, longest) / 2;  // over a sequence's items
+  double rounds = (double)generic / kCUs;
+  // mostly cached tokens: items of about one length, so whole rounds
+  if (longest > 2 * (p.batch == 1 ? mean : (double)p.max_seqlen_q)) rounds = std::ceil(rounds);
+  const double t_generic = std::max(12 + .044 * longest, rounds * (12 + .044 * average) + (generic > kCUs ? 4 : 0));
+  const double t_tiled = std::max(10 + .057 * longest, (double)tiled / kCUs * (10 + .057 * average));
+  return t_tiled < t_generic;
+}
+
 bool prefill_tiled(const PrefillParams& p, int head_dim) {
   if (p.batch == 0 || p.max_seqlen_q == 0) return false;
-  const int64_t tile_tokens = kRows / p.group;
-  const int64_t pairs = p.batch * ((p.max_seqlen_q + tile_tokens - 1) / tile_tokens);
-  // At 256 the generic kernel's items are half as long (128 rows): while they
-  // fit one round on the CUs it is faster (3 x 299 tokens, 32 / 8 heads, 29.1
-  // us against 31.7; 2 x 300 behind 4000 cached 203 against 260), from there
-  // on this one (4 x 511 tokens 47 us against 52, 8 x 512 64 against 96).
-  const int64_t live = std::min<int64_t>(pairs, p.num_tokens / tile_tokens + p.batch);
   switch (head_dim) {
     case 64: return paging_of<64>(p) != kPageLane;
     case 96: return paging_of<96>(p) != kPageLane;
-    case 256: return p.group <= 128 && paging_of<256>(p) != kPageLane && live * p.num_kv_heads >= kCUs / 2;
+    case 256: return p.group <= 128 && paging_of<256>(p) != kPageLane && tiled_256_pays(p);
     default: return false;
   }
 }
