@@ -434,6 +434,9 @@ def test_prefill_page_sizes_bit_identical(pkg, dev, prefix):
     ([3000], [1], 8, 1, 64, None),                        # one row, one kv head: 8 q rows, many parts
     ([0], [1999], 16, 8, 16, None),                       # a fresh prompt: only its long items split
     ([1600, 1, 0, 5], [0, 3, 128, 129], 12, 3, 32, None),  # a sequence without rows, 3 kv heads
+    ([1600, 2500, 5, 900], [70, 0, 129, 100], 12, 3, 32, None),  # real parts at 3 kv heads, whose share does not divide
+    ([0, 3000, 0], [300, 40, 500], 16, 1, 64, None),       # one kv head, 16-token tiles: 96 pairs
+    ([0], [2500], 16, 1, 64, None),                        # as many pairs as there can be
 ])
 def test_prefill_split_items(pkg, dev, prefix, new, h, hkv, bs, cap):
     """Launches of few, long items split them over their kv range: the oracle,

@@ -62,23 +62,6 @@ constexpr int kDecodeMinChunk = 512;   // shortest item of a small launch
 // 32-token pages whole pages (a 2048-token part then spans 64 of them).
 __host__ __device__ inline int balance_align(int page_size) { return page_size == 32 ? 32 : 16; }
 
-// Inclusive prefix sum over the wave's lanes: shifts inside the rows of 16
-// lanes, then the row totals broadcast to the rows above (DPP; the LDS
-// permutes of __shfl_up cost ten times the latency on this serial path).
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ uint32_t scan_dpp(uint32_t x) {
-  return x + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, kRowMask, 0xF, false);
-}
-__device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
-  x = scan_dpp<0x111, 0xF>(x);  // row_shr:1
-  x = scan_dpp<0x112, 0xF>(x);  // row_shr:2
-  x = scan_dpp<0x114, 0xF>(x);  // row_shr:4
-  x = scan_dpp<0x118, 0xF>(x);  // row_shr:8
-  x = scan_dpp<0x142, 0xA>(x);  // row_bcast:15 into rows 1 and 3
-  x = scan_dpp<0x143, 0xC>(x);  // row_bcast:31 into rows 2 and 3
-  return x;
-}
-
 // ceil(x / d) for 0 <= x < 2^23, 0 < d < 2^23: a float quotient, put right.
 __device__ __forceinline__ int ceil_div_small(int x, int d) {
   int q = (int)((float)x * __builtin_amdgcn_rcpf((float)d));

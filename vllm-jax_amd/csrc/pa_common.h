@@ -156,6 +156,23 @@ __device__ __forceinline__ float soft_cap_s2(float logit_scale, float cap) {
 }
 __device__ __forceinline__ float soft_cap_c(float cap) { return cap * kLog2e; }
 
+// Inclusive prefix sum over the wave's lanes: shifts inside the rows of 16
+// lanes, then the row totals broadcast to the rows above (DPP; the LDS
+// permutes of __shfl_up cost ten times the latency on this serial path).
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ uint32_t scan_dpp(uint32_t x) {
+  return x + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, kRowMask, 0xF, false);
+}
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
+  x = scan_dpp<0x111, 0xF>(x);  // row_shr:1
+  x = scan_dpp<0x112, 0xF>(x);  // row_shr:2
+  x = scan_dpp<0x114, 0xF>(x);  // row_shr:4
+  x = scan_dpp<0x118, 0xF>(x);  // row_shr:8
+  x = scan_dpp<0x142, 0xA>(x);  // row_bcast:15 into rows 1 and 3
+  x = scan_dpp<0x143, 0xC>(x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
 // Exclusive scan over the workgroup (blockDim.x == kScanThreads) of one
 // value per thread; `tmp` is kScanThreads ints of LDS.  Returns the sum of
 // the values of lower threads; `total` receives the sum of all.

@@ -83,8 +83,9 @@ struct PrefillParams {
   // Work list (may be null): plan[0] = number of (sequence, q tile) pairs with
   // rows, PrefillPair records from int kPlanHeader on, most kv tiles first.
   const int32_t* plan;
-  // Launches that split items over the kv range (prefill_split.hip): a record
-  // (parts, first slot, q0, rows) per (sequence, q tile) pair, and the partials.
+  // Launches that split items over the kv range (prefill_split.hip): the
+  // number of split (sequence, q tile) pairs, a record (parts and q tile, first
+  // slot, q0, rows) for each, and the partials.
   int32_t* split;
   float* parts;
   // With the work list and num_kv_heads % 8 == 0: the counters of the eight

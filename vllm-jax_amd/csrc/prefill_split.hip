@@ -6,9 +6,9 @@
 // Here every workgroup first counts the launch's kv tiles (one thread per
 // (sequence, q tile) pair, as prefill_plan estimates them), finds a part
 // length with which the parts fill the chip once, and runs one part of one
-// item, longest parts first.  A part leaves its unnormalised O, reference max
+// item.  A part leaves its unnormalised O, reference max
 // and row sums in f32; prefill_split_merge_kernel adds the parts up.  That
-// call: 226 us unsplit, 89.7 + 8.0 us so (131 with parts of an even share,
+// call: 217 us unsplit, 92 us so (131 with parts of an even share,
 // whose 288 parts took two rounds).  What is left: about 1.1 us a tile and 10
 // us around the loop, and 32 MB of partials written and read.
 #include <algorithm>
@@ -21,9 +21,9 @@ namespace pa {
 namespace {
 
 constexpr int kSplitCUs = 256;
-// Pairs the in-kernel count takes: each of up to 256 threads compares its pair
-// with all others.
+// Pairs the in-kernel count takes.
 constexpr int kSplitMaxPairs = 256;
+static_assert(kSplitMaxPairs % 64 == 0 && kSplitMaxPairs <= kThreads, "one thread per pair, whole waves");
 // No part below this many tiles is made: a part costs about 7 us outside its
 // loop, and a tile about 1 us.
 constexpr int kSplitMinTiles = 8;
@@ -37,15 +37,18 @@ constexpr int64_t kSplitMaxItems = kSplitCUs;
 // Largest grid (n_qtiles x batch x kv heads) that is looked at.
 constexpr int64_t kSplitMaxGrid = 1024;
 
-// Parts and slots of a launch: sum over pairs of ceil(tiles / L) with L at
+// Slots of a launch: sum over pairs of ceil(tiles / L) with L at
 // least an even share, tiles * kv heads / kSplitCUs, is at most kSplitCUs / kv
 // heads + pairs; only split pairs (two parts or more, so longer than L, so at
 // most kSplitCUs / kv heads of them) take slots.
-int64_t split_max_parts(int64_t pairs, int32_t hkv) { return kSplitCUs / hkv + pairs; }
 int64_t split_max_slots(int64_t pairs, int32_t hkv) {
   const int64_t share = kSplitCUs / hkv;
-  return (share + (pairs < share ? pairs : share)) * hkv;
+  return (share + std::min(pairs, share)) * hkv;
 }
+// Split pairs of a launch: longer than L, so fewer than kSplitCUs / kv heads.
+int64_t split_max_pairs(int64_t pairs, int32_t hkv) { return std::min<int64_t>(pairs, kSplitCUs / hkv); }
+// The number of split pairs, then a record of four ints for each (fewer than
+// 256, so that the number and they fit).
 constexpr size_t kSplitHeader = kSplitMaxPairs * 4 * sizeof(int32_t);
 
 template <bool kSoftCap, int kPaging>
@@ -56,9 +59,13 @@ prefill_split_kernel(PrefillParams p, int grid_parts) {
     return;
   }
   __shared__ unsigned long long s_total;
-  __shared__ int32_t s_tiles[kSplitMaxPairs], s_size[kSplitMaxPairs], s_parts[kSplitMaxPairs];
-  __shared__ int32_t s_work[12];
+  __shared__ int32_t s_tiles[kSplitMaxPairs];
+  __shared__ float s_count[kWaves][64];
+  __shared__ uint32_t s_before[kSplitMaxPairs / 64];
+  __shared__ int32_t s_work[9];
   const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hkv = p.num_kv_heads;
   const int nq = p.n_qtiles;
   const int pairs = p.batch * nq;
@@ -77,57 +84,63 @@ prefill_split_kernel(PrefillParams p, int grid_parts) {
     prefill_seq_geometry(p, b, g, lag);
     tiles = prefill_pair_tiles(g, lag, qt, p.tile_tokens);  // -1: no rows
     if (tiles > 0) atomicAdd(&s_total, (unsigned long long)tiles);
-    s_tiles[tid] = tiles;
   }
+  if (tid < kSplitMaxPairs) s_tiles[tid] = tiles;
   __syncthreads();
   // The part length: an even share of the launch's tiles leaves more parts
   // than CUs (every pair rounds up), so lane k of each wave counts the parts
-  // at a share times 1 + k / 16 and the shortest length that fits one round
-  // is taken (the even share if none does).
+  // of the wave's share of the pairs at a share times 2^(k / 10), and the
+  // shortest length that fits one round is taken.  If none does (one pair 78
+  // times the share, or more), nothing is split.
   const int64_t share = ((int64_t)s_total * hkv + kSplitCUs - 1) / kSplitCUs;
-  const int lane = tid & 63;
-  const int64_t least = max((int64_t)kSplitMinTiles, share);
-  const int cand = (int)min(least + least * lane / 16, (int64_t)INT_MAX);
-  const float inv = 1.f / (float)cand;
+  const float cand = ceilf((float)max((int64_t)kSplitMinTiles, share) * exp2f(.1f * (float)lane));
+  const float inv = 1.f / cand;
   float count = 0.f;
-  for (int j = 0; j < pairs; ++j) {
+  const int per_wave = (pairs + kWaves - 1) / kWaves;
+#pragma unroll 4
+  for (int j = wave * per_wave; j < min(pairs, (wave + 1) * per_wave); ++j) {
     const float tj = (float)s_tiles[j];
     count += tj < 0.f ? 0.f : fmaxf(1.f, ceilf(tj * inv));
   }
-  const uint64_t fits = __ballot(count * (float)hkv <= (float)kSplitCUs);
-  const int len = __shfl(cand, fits ? __ffsll((unsigned long long)fits) - 1 : 0);
-  const int parts = tiles < 0 ? 0 : max(1, (int)(((int64_t)tiles + len - 1) / len));
-  const int size = parts ? (tiles + parts - 1) / parts : -1;
-  if (tid < kSplitMaxPairs) {
-    s_size[tid] = size;
-    s_parts[tid] = parts;
-  }
+  s_count[wave][lane] = count;
   __syncthreads();
-  if (tid < pairs && parts) {
-    int at = 0, slot = 0;  // parts listed before this pair's, and partials
-    for (int j = 0; j < pairs; ++j) {
-      const int sj = s_size[j], pj = s_parts[j];
-      const bool before = sj > size || (sj == size && j < tid);
-      at += before ? pj : 0;
-      slot += before && pj > 1 ? pj : 0;
-    }
-    if (mine >= at && mine < at + parts) {
-      const int k = mine - at;
-      s_work[0] = b;
-      s_work[1] = qt;
-      s_work[2] = g.x;
-      s_work[3] = g.y;
-      s_work[4] = g.z;
-      s_work[5] = g.w;
-      s_work[6] = (int)((int64_t)tiles * k / parts);
-      s_work[7] = k + 1 == parts ? INT_MAX : (int)((int64_t)tiles * (k + 1) / parts);
-      s_work[8] = parts > 1 ? (slot + k) * hkv : -1;
-    }
-    if (blockIdx.x == 0) {  // for the merge
-      st16(p.split + 4 * tid, u32x4{(uint32_t)parts, (uint32_t)(slot * hkv), (uint32_t)g.x, (uint32_t)g.y});
-    }
-  } else if (tid < pairs && blockIdx.x == 0) {
-    p.split[4 * tid] = 0;
+  count = 0.f;
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) count += s_count[i][lane];
+  const uint64_t fits = __ballot(count * (float)hkv <= (float)kSplitCUs);
+  const float len = fits ? __shfl(cand, __ffsll((unsigned long long)fits) - 1) : (float)INT_MAX;
+  const int parts = tiles < 0 ? 0 : max(1, (int)ceilf((float)tiles * (1.f / len)));  // as counted
+  // parts, partial slots and split pairs of the pairs before this one, ten
+  // bits each: at most kSplitCUs of them
+  const uint32_t own = (uint32_t)parts | (parts > 1 ? (uint32_t)parts << 10 | 1u << 20 : 0u);
+  uint32_t upto = wave_scan(own);
+  if (lane == 63 && wave < kSplitMaxPairs / 64) s_before[wave] = upto;
+  __syncthreads();
+  uint32_t all = 0;
+#pragma unroll
+  for (int i = 0; i < kSplitMaxPairs / 64; ++i) {
+    upto += i < wave ? s_before[i] : 0;
+    all += s_before[i];
+  }
+  const uint32_t before = upto - own;
+  const int at = (int)(before & 0x3ff), slot = (int)(before >> 10 & 0x3ff);
+  if (mine >= at && mine < at + parts) {
+    const int k = mine - at;
+    s_work[0] = b;
+    s_work[1] = qt;
+    s_work[2] = g.x;
+    s_work[3] = g.y;
+    s_work[4] = g.z;
+    s_work[5] = g.w;
+    s_work[6] = (int)((int64_t)tiles * k / parts);
+    s_work[7] = k + 1 == parts ? INT_MAX : (int)((int64_t)tiles * (k + 1) / parts);
+    s_work[8] = parts > 1 ? (slot + k) * hkv : -1;
+  }
+  if (blockIdx.x == 0) {  // for the merge
+    if (tid == 0) p.split[0] = (int)(all >> 20);
+    if (parts > 1)
+      st16(p.split + 4 * (1 + (before >> 20)), u32x4{(uint32_t)parts | (uint32_t)qt << 16, (uint32_t)(slot * hkv),
+                                                     (uint32_t)g.x, (uint32_t)g.y});
   }
   __syncthreads();
   auto work = [&](int i) { return __builtin_amdgcn_readfirstlane(s_work[i]); };
@@ -150,25 +163,25 @@ prefill_split_kernel(PrefillParams p, int grid_parts) {
 
 // out = sum_k o_k 2^(m_k - M) / sum_k l_k 2^(m_k - M) over an item's parts k,
 // M their largest reference max.
-// One workgroup per (pair, kv head, 32-row block), one wave per 32 d: the
+// One workgroup per (split pair, kv head, 32-row block), one wave per 32 d: the
 // lanes hold what the part's accumulators held.
 __global__ void __launch_bounds__(256)
 prefill_split_merge_kernel(PrefillParams p) {
   const int hkv = p.num_kv_heads;
   const int item = blockIdx.x / kWaves;
   const int block = blockIdx.x - item * kWaves;
-  const int pair = item / hkv;
-  const int kvh = item - pair * hkv;
-  const int4 rec = *reinterpret_cast<const int4*>(p.split + 4 * pair);  // parts, first slot, q0, rows
-  const int parts = rec.x;
-  if (parts < 2) return;
+  const int rank = item / hkv;
+  const int kvh = item - rank * hkv;
+  if (rank >= p.split[0]) return;
+  const int4 rec = *reinterpret_cast<const int4*>(p.split + 4 * (1 + rank));  // parts and q tile, first slot, q0, rows
+  const int parts = rec.x & 0xffff;
   const float* src = p.parts + (int64_t)(rec.y + kvh) * kPartFloats<kPHeadDim>;
   const int64_t step = (int64_t)hkv * kPartFloats<kPHeadDim>;
   const int lane = threadIdx.x & 63;
   const int dt = threadIdx.x >> 6;
   const int n = lane & 31, h = lane >> 5;
   const int row = 32 * block + n;
-  const int rtok = (pair - pair / p.n_qtiles * p.n_qtiles) * p.tile_tokens + row / p.group;
+  const int rtok = (rec.x >> 16) * p.tile_tokens + row / p.group;
   const float* ml = src + kPartO<kPHeadDim> + 2 * row;
   const float* po = src + 4 * ((block * 4 + dt) * 4 * 64 + lane);
   f32x4 o[4] = {};
@@ -217,7 +230,8 @@ int prefill_split_launch(const char* name, const PrefillParams& prm, int paging,
   p.split = reinterpret_cast<int32_t*>(workspace);
   p.parts = reinterpret_cast<float*>((char*)workspace + kSplitHeader);
   const int64_t pairs = (int64_t)p.batch * p.n_qtiles;
-  const int grid_parts = (int)(split_max_parts(pairs, p.num_kv_heads) * p.num_kv_heads);
+  // the parts fit one round, and so do the pairs with rows (prefill_splits)
+  const int grid_parts = kSplitCUs / p.num_kv_heads * p.num_kv_heads;
   // workgroups past the parts zero the rows no item writes, 512 tokens each
   const int64_t blocks = grid_parts + ((int64_t)p.num_tokens + kThreads - 1) / kThreads;
   const dim3 grid((unsigned)blocks), blk(kThreads);
@@ -231,7 +245,8 @@ int prefill_split_launch(const char* name, const PrefillParams& prm, int paging,
   else launch(std::false_type{});
   const int rc = launch_status(name);
   if (rc) return rc;
-  prefill_split_merge_kernel<<<dim3((unsigned)(pairs * p.num_kv_heads * kWaves)), dim3(256), 0, s>>>(p);
+  const int64_t merges = split_max_pairs(pairs, p.num_kv_heads) * p.num_kv_heads * kWaves;
+  if (merges > 0) prefill_split_merge_kernel<<<dim3((unsigned)merges), dim3(256), 0, s>>>(p);
   return launch_status(name);
 }
 
