@@ -196,13 +196,16 @@ size_t pa_prefill_split_workspace_size(int32_t batch, int32_t max_seqlen_q, int3
                                        int32_t head_dim, int32_t pages_per_seq, int32_t page_size);
 
 /* Which kernel a pa_prefill launch of this shape runs (bf16 pages whose rows
- * are num_kv_heads * head_dim apart): PA_PREFILL_GENERIC or PA_PREFILL_TILED,
- * or PA_ERR_INVALID_ARGUMENT for bad sizes.  cached: cu_seqlens_k is given and
+ * are num_kv_heads * head_dim apart): PA_PREFILL_GENERIC, PA_PREFILL_TILED, or
+ * PA_PREFILL_SPLIT (tiled, the long items split over their kv range, if the
+ * workspace has pa_prefill_split_workspace_size bytes), or
+ * PA_ERR_INVALID_ARGUMENT for bad sizes.  cached: cu_seqlens_k is given and
  * is not cu_seqlens_q, so that tokens before the new ones may be in the pages.
  * No device is touched.  No counterpart in the reference, which has one
  * kernel. */
 #define PA_PREFILL_GENERIC 0
 #define PA_PREFILL_TILED 1
+#define PA_PREFILL_SPLIT 2
 int pa_prefill_route(int32_t batch, int32_t num_tokens, int32_t max_seqlen_q, int32_t num_heads, int32_t num_kv_heads,
                      int32_t head_dim, int32_t pages_per_seq, int32_t page_size, int32_t cached);
 

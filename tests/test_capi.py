@@ -391,3 +391,42 @@ def test_prefill_route_edges():
         assert route(*bad) == -1
     for empty in ((0, 0, 0), (0, 5, 0), (1, 0, 100), (1, 5, 0)):
         assert route(*empty, 32, 8, 256, 0, 256, 1) in (0, 1)
+
+
+@pytest.mark.parametrize("new,prefix,heads,hkv,split", [
+    # timed faster with the long items split (exact tables, 256-token pages)
+    ([400, 128], 15000, 32, 8, True), ([64], 1500, 32, 8, True), ([300], 1500, 32, 8, True),
+    ([100] * 4, 1500, 32, 8, True), ([800], 8000, 32, 8, True), ([1500], 8000, 16, 8, True),
+    ([400] * 3, 2000, 16, 8, True), ([2400], 0, 16, 8, True), ([2000], 0, 16, 8, True),
+    ([1700, 64], 16000, 32, 8, True), ([2200], 0, 16, 1, True),
+    # timed slower, or within 2 %
+    ([1600], 0, 32, 8, False), ([1792], 0, 32, 8, False), ([1984], 0, 32, 8, False), ([2040], 0, 32, 8, False),
+    ([3300], 0, 16, 8, False), ([3700], 0, 16, 8, False), ([3968], 0, 16, 8, False),
+    ([1100], 8000, 32, 8, False), ([1500], 8000, 32, 8, False), ([1900], 8000, 32, 8, False),
+    ([2500], 8000, 16, 8, False), ([400] * 3, 2000, 32, 8, False), ([1000], 1000, 32, 8, False),
+    ([800], 500, 32, 8, False), ([100], 0, 32, 8, False), ([900] * 2, 0, 32, 8, False),
+])
+def test_prefill_route_splits_where_it_pays(new, prefix, heads, hkv, split):
+    """Whether a launch of few items is split (prefill_split.hip)."""
+    route = PKG._lib.load().pa_prefill_route
+    bucket = 1 << (max(new) - 1).bit_length()
+    pages = -(-(max(new) + prefix) // 256)
+    assert route(len(new), sum(new), bucket, heads, hkv, 128, pages, 256, 1) == 1 + split
+    # nothing cached, in a table for 32k tokens: the new tokens bound the kv lengths
+    if not prefix:
+        assert route(len(new), sum(new), bucket, heads, hkv, 128, 128, 256, 0) == 1 + split
+
+
+def test_prefill_split_grid_holds_every_pair():
+    """A launch that splits has fewer items than CUs whatever its sequences
+    are, so that one round of workgroups holds every pair with rows."""
+    route = PKG._lib.load().pa_prefill_route
+    for heads, hkv in ((32, 8), (16, 8), (64, 8), (8, 8), (64, 2), (16, 1), (12, 3), (40, 40), (300, 300)):
+        tile = 256 // (heads // hkv)
+        for batch in (1, 2, 3, 8, 40):
+            for tokens in (batch, 100 * batch, 700 * batch, 2500 * batch):
+                if route(batch, tokens, 4096, heads, hkv, 128, 2048, 16, 1) != 2:
+                    continue
+                # most pairs: every sequence but one has a single token in its last tile
+                pairs = sum(-(-n // tile) for n in [tokens - (batch - 1)] + [1] * (batch - 1))
+                assert pairs <= 256 // hkv

@@ -451,6 +451,8 @@ def test_prefill_split_items(pkg, dev, prefix, new, h, hkv, bs, cap):
     split = lib.pa_prefill_split_workspace_size(pb.batch, int(pb.max_seqlen_bucket), h, hkv, 128,
                                                 pb.block_tables.shape[1], bs)
     assert split > plan + 4 * 128 * 256
+    assert lib.pa_prefill_route(pb.batch, int(pb.cu_seqlens_q[-1]), int(pb.max_seqlen_bucket), h, hkv, 128,
+                                pb.block_tables.shape[1], bs, 1) == 2
     got, t = _prefill(pkg, dev, pb, seed=7, soft_cap=cap, use_seam=False)
     args = (t["q"], t["kv_cache"][0].permute(2, 0, 1, 3), t["kv_cache"][1].permute(2, 0, 1, 3), t["block_tables"],
             t["cu_seqlens_q"], t["slot_mapping"], t["input_positions"])
@@ -461,6 +463,34 @@ def test_prefill_split_items(pkg, dev, prefix, new, h, hkv, bs, cap):
     ws = torch.full((split,), 255, dtype=torch.uint8, device=dev)
     two = pkg.prefill_paged_attention(*args, workspace=ws, **kw)
     assert np.array_equal(ora.bf16_to_f32(u16(two)), got)
+
+
+def test_prefill_split_only_where_it_pays(pkg, dev):
+    """A prompt that a split would not make faster is not given the partials'
+    68 MB; equal items that only a second round of parts would shorten are left
+    whole by the kernel: bit for bit the unsplit launch."""
+    import torch
+
+    def peak_and_out(prefix, new, workspace=None):
+        pb = wl.make_prefix_prefill(prefix, new, num_heads=32, num_kv_heads=8, page_size=256,
+                                    rng=np.random.default_rng(5), shared_prefix_tokens=0)
+        t = wl.materialize_prefill(pb, 3, dev, fill_pool=True)
+        out = torch.empty_like(t["q"])
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        pkg.prefill_paged_attention(
+            t["q"], t["kv_cache"][0].permute(2, 0, 1, 3), t["kv_cache"][1].permute(2, 0, 1, 3), t["block_tables"],
+            t["cu_seqlens_q"], t["slot_mapping"], t["input_positions"], max_seqlen_bucket=pb.max_seqlen_bucket,
+            cu_seqlens_k=t["cu_seqlens_k"], out=out, workspace=workspace)
+        return torch.cuda.max_memory_allocated() - before, out
+
+    assert peak_and_out([0], [1999])[0] < 1 << 20
+    assert peak_and_out([6000, 9000], [200, 100])[0] > 8 << 20
+    need, whole = peak_and_out([6000] * 3, [600] * 3)
+    assert need > 8 << 20  # the host cannot tell
+    listed = torch.empty(1 << 16, dtype=torch.uint8, device=dev)
+    assert torch.equal(whole, peak_and_out([6000] * 3, [600] * 3, listed)[1])
 
 
 def test_prefill_split_rows_without_keys_and_rows_past_the_bucket(pkg, dev):

@@ -566,7 +566,9 @@ extern "C" int pa_prefill_route(int32_t batch, int32_t num_tokens, int32_t max_s
   p.tile_tokens = kRows / p.group;
   p.n_qtiles = (max_seqlen_q + p.tile_tokens - 1) / p.tile_tokens;
   if (head_dim != kPHeadDim) return prefill_tiled(p, head_dim) ? PA_PREFILL_TILED : PA_PREFILL_GENERIC;
-  return PA_PREFILL_TILED;
+  return prefill_splits(p) && prefill_split_bytes(batch, p.n_qtiles, num_kv_heads, (int64_t)pages_per_seq * page_size)
+             ? PA_PREFILL_SPLIT
+             : PA_PREFILL_TILED;
 }
 #endif
 

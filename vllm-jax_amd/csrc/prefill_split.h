@@ -12,7 +12,8 @@ struct PrefillParams;
 // shape is not one that splits.  span: tokens a block-table row can hold.
 size_t prefill_split_bytes(int32_t batch, int32_t n_qtiles, int32_t num_kv_heads, int64_t span);
 
-// Whether a launch of `p` has few enough items to be split.
+// Whether a launch of `p` (head size 128) has few enough, long enough items for
+// a split to pay.
 bool prefill_splits(const PrefillParams& p);
 
 // Split launch of `p` (head size 128, bf16 pages) with a workspace of

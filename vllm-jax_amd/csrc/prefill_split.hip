@@ -11,6 +11,13 @@
 // call: 217 us unsplit, 92 us so (131 with parts of an even share,
 // whose 288 parts took two rounds).  What is left: about 1.1 us a tile and 10
 // us around the loop, and 32 MB of partials written and read.
+//
+// A split pays where the parts are shorter than the longest item by more than
+// the count, the partials and the merge cost.  The kernel knows the lengths
+// and splits nothing where it does not; the host knows an upper bound of the
+// items and takes the longest kv length from the table's width (from the new
+// tokens where cu_seqlens_k says that nothing is cached), and launches the
+// plain kernel where a split cannot be told to pay (prefill_splits).
 #include <algorithm>
 #include <climits>
 
@@ -27,13 +34,25 @@ static_assert(kSplitMaxPairs % 64 == 0 && kSplitMaxPairs <= kThreads, "one threa
 // No part below this many tiles is made: a part costs about 7 us outside its
 // loop, and a tile about 1 us.
 constexpr int kSplitMinTiles = 8;
-// Shortest table span (in kv tiles) that is worth the merge launch.
+// Shortest table span (in kv tiles) of a launch that splits.
 constexpr int kSplitMinSpan = 24;
-// Bound on the items (pairs with rows x kv heads) of a launch that splits.
-// From a CU's worth on the parts need a second round, each with its own fixed
-// cost, and the merge: one 1 999-token prompt (256 items of 1 to 32 tiles,
-// Qwen3-8B heads) took 52 us unsplit and 55 + 10 us split.
-constexpr int64_t kSplitMaxItems = kSplitCUs;
+// From this longest kv length (in tiles) on several sequences are looked at by
+// the kernel even where equal ones would gain nothing.  Where it then splits
+// nothing, the count and the merge launch cost 4 to 7 us of 105 to 240; where
+// it splits, such launches gain 20 % on average and up to 70.
+constexpr int kSplitTryLongest = 80;
+// Items that run at an item's own speed; more share the chip's power (a kv
+// tile takes 1.04 us with up to 150 items at once, 1.45 us with 240).
+constexpr float kSplitBusy = 165.f;
+// What a split costs, in tiles: the count, the partials, the merge.
+constexpr float kSplitCost = 9.f;
+// Time, in tiles, of `parts` parts of `total` tiles in all, the longest of
+// `len`: all but the longest as if they ended together.
+__host__ __device__ inline float split_time(float len, float parts, float total) {
+  return parts <= kSplitBusy ? len : fmaxf(len, total / kSplitBusy + len - total / parts);
+}
+// At least the time of the launch unsplit.
+__host__ __device__ inline float whole_time(float longest, float total) { return fmaxf(longest, total / kSplitBusy); }
 // Largest grid (n_qtiles x batch x kv heads) that is looked at.
 constexpr int64_t kSplitMaxGrid = 1024;
 
@@ -60,7 +79,7 @@ prefill_split_kernel(PrefillParams p, int grid_parts) {
   }
   __shared__ unsigned long long s_total;
   __shared__ int32_t s_tiles[kSplitMaxPairs];
-  __shared__ float s_count[kWaves][64];
+  __shared__ float s_count[kWaves][64], s_longest[kWaves];
   __shared__ uint32_t s_before[kSplitMaxPairs / 64];
   __shared__ int32_t s_work[9];
   const int tid = threadIdx.x;
@@ -95,20 +114,31 @@ prefill_split_kernel(PrefillParams p, int grid_parts) {
   const int64_t share = ((int64_t)s_total * hkv + kSplitCUs - 1) / kSplitCUs;
   const float cand = ceilf((float)max((int64_t)kSplitMinTiles, share) * exp2f(.1f * (float)lane));
   const float inv = 1.f / cand;
-  float count = 0.f;
+  float count = 0.f, longest = 0.f;
   const int per_wave = (pairs + kWaves - 1) / kWaves;
 #pragma unroll 4
   for (int j = wave * per_wave; j < min(pairs, (wave + 1) * per_wave); ++j) {
     const float tj = (float)s_tiles[j];
     count += tj < 0.f ? 0.f : fmaxf(1.f, ceilf(tj * inv));
+    longest = fmaxf(longest, tj);
   }
   s_count[wave][lane] = count;
+  s_longest[wave] = longest;  // the same in every lane
   __syncthreads();
   count = 0.f;
 #pragma unroll
-  for (int i = 0; i < kWaves; ++i) count += s_count[i][lane];
+  for (int i = 0; i < kWaves; ++i) {
+    count += s_count[i][lane];
+    longest = fmaxf(longest, s_longest[i]);
+  }
   const uint64_t fits = __ballot(count * (float)hkv <= (float)kSplitCUs);
-  const float len = fits ? __shfl(cand, __ffsll((unsigned long long)fits) - 1) : (float)INT_MAX;
+  float len = (float)INT_MAX;
+  if (fits) {
+    const int first = __ffsll((unsigned long long)fits) - 1;
+    const float at = __shfl(cand, first), total = (float)s_total * (float)hkv;
+    const float split = split_time(at, __shfl(count, first) * (float)hkv, total) + kSplitCost;
+    if (split < whole_time(longest, total)) len = at;
+  }
   const int parts = tiles < 0 ? 0 : max(1, (int)ceilf((float)tiles * (1.f / len)));  // as counted
   // parts, partial slots and split pairs of the pairs before this one, ten
   // bits each: at most kSplitCUs of them
@@ -219,10 +249,39 @@ size_t prefill_split_bytes(int32_t batch, int32_t n_qtiles, int32_t num_kv_heads
   return kSplitHeader + (size_t)split_max_slots(pairs, num_kv_heads) * kPartFloats<kPHeadDim> * sizeof(float);
 }
 
+// With N items, the longest of T tiles (N an upper bound, T a lower one), a
+// split surely pays if it does where every sequence is as long as the longest:
+// to bring that down to L tiles each sequence has at most 64 (T - L) /
+// tile_tokens items a kv head cut in two; or all N items are cut in 256 / N.
+// Unsplit -> split, 32 / 8 heads unless said, us: 64 new tokens behind 1500
+// cached 35.4 -> 22.4, 4 x 100 behind 1500 36.0 -> 30.4, 800 behind 8000 153.6
+// -> 111.5, fresh 2400 at 16 / 8 heads 50.4 -> 43.8.  Split before this rule,
+// and slower: fresh 1792 41.9 -> 47.7, fresh 3500 at 16 / 8 heads 72.0 -> 77.0,
+// 1100 behind 8000 160.9 -> 178.9, 3 x 400 behind 2000 54.7 -> 60.5.
 bool prefill_splits(const PrefillParams& p) {
-  // pairs with rows: a sequence of n tokens has ceil(n / tile_tokens)
-  const int64_t live = std::min<int64_t>((int64_t)p.batch * p.n_qtiles, p.num_tokens / p.tile_tokens + p.batch);
-  return live * p.num_kv_heads < kSplitMaxItems;
+  const int64_t tile = p.tile_tokens, batch = p.batch, hkv = p.num_kv_heads;
+  if (batch == 0 || p.n_qtiles == 0 || batch * p.n_qtiles * hkv >= kSplitMaxGrid) return false;
+  // pairs with rows: a sequence of n tokens has ceil(n / tile)
+  const int64_t items = std::min<int64_t>(batch * p.n_qtiles, (p.num_tokens + batch * (tile - 1)) / tile) * hkv;
+  if (items == 0 || items >= kSplitCUs) return false;
+  const int64_t span = (int64_t)p.pages_per_seq * p.page_size, mean = (p.num_tokens + batch - 1) / batch;
+  const bool fresh = !p.cu_k || p.cu_k == p.cu_q;
+  const int64_t kv = fresh ? std::min(span, mean) : std::max(span - p.page_size + 1, mean);
+  const int64_t longest = (kv + kTileN - 1) / kTileN;
+  if (longest == 0) return false;
+  const float t = (float)longest, n = (float)items;
+  // the items of a sequence are tile / 64 tiles apart
+  const float total = n * std::max(.5f * t, t - (n / (float)(batch * hkv) - 1.f) * (float)tile / (2 * kTileN));
+  // (one cost more than the kernel's: the bounds round to whole tiles)
+  const float whole = (batch == 1 ? whole_time(t, total) : t) - kSplitCost - 1.f;
+  const float step = (float)(batch * kTileN * hkv) / (float)tile;
+  const float half = std::max(.5f * t, t - ((float)kSplitCUs - n) / step);
+  if (half < t && split_time(std::max(half, (float)kSplitMinTiles), n + std::min(n, step * (t - half)), total) < whole)
+    return true;
+  const int64_t ways = kSplitCUs / items;
+  const int64_t len = std::max<int64_t>(kSplitMinTiles, (longest + ways - 1) / ways);
+  if (split_time((float)len, n * (float)((longest + len - 1) / len), total) < whole) return true;
+  return batch > 1 && longest >= kSplitTryLongest;
 }
 
 int prefill_split_launch(const char* name, const PrefillParams& prm, int paging, void* workspace, hipStream_t s) {

@@ -22,6 +22,8 @@ from .. import _lib
 from ._common import (DEFAULT_MASK_VALUE, as_i32, check_quantized_pages, inv_sqrt_head_dim_bf16, pages_strides,
                       pool_pointers, require_bf16, require_device, stream_handle)
 
+_ROUTE_SPLIT = 2  # PA_PREFILL_SPLIT
+
 
 def prefill_paged_attention(
         q: torch.Tensor,
@@ -160,8 +162,11 @@ def _prefill(q, pages, pointers, strides, code_type, scales, block_tables, cu_se
                                                       int(max_seqlen_bucket), num_heads)) - need
     if workspace is None or workspace.numel() * workspace.element_size() < need + extra:
         # our own: with room for the parts of a launch that splits its items
-        need = int(lib.pa_prefill_split_workspace_size(batch, int(max_seqlen_bucket), num_heads, num_kv_heads,
-                                                       head_dim, pages_per_sequence, page_size))
+        cached = cuk is not None and cuk.data_ptr() != cu.data_ptr()
+        if lib.pa_prefill_route(batch, total_tokens, int(max_seqlen_bucket), num_heads, num_kv_heads, head_dim,
+                                pages_per_sequence, page_size, cached) == _ROUTE_SPLIT:
+            need = int(lib.pa_prefill_split_workspace_size(batch, int(max_seqlen_bucket), num_heads, num_kv_heads,
+                                                           head_dim, pages_per_sequence, page_size))
         workspace = torch.empty(max(need + extra, 1), dtype=torch.uint8, device=q.device)
     ws_bytes = workspace.numel() * workspace.element_size()
     if quantized:
