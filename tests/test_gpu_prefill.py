@@ -493,6 +493,39 @@ def test_prefill_split_only_where_it_pays(pkg, dev):
     assert torch.equal(whole, peak_and_out([6000] * 3, [600] * 3, listed)[1])
 
 
+def test_prefill_split_follows_the_longest_kv_length(pkg, dev):
+    """In a table for 32k tokens max_seqlen_k says whether a split can pay:
+    without partials, short prompts are bit for bit the unsplit launch."""
+    import torch
+    pb = wl.make_prefix_prefill([0, 0], [200, 100], num_heads=32, num_kv_heads=8, page_size=256,
+                                rng=np.random.default_rng(6), shared_prefix_tokens=0)
+    t = wl.materialize_prefill(pb, 4, dev, fill_pool=True)
+    table = torch.full((2, 128), -1, dtype=torch.int32, device=dev)
+    table[:, :t["block_tables"].shape[1]] = t["block_tables"]
+
+    def run(max_seqlen_k, cu_k):
+        meta = pkg.PrefillAttentionMetadata(t["input_positions"], t["slot_mapping"], table, t["cu_seqlens_q"], cu_k, None,
+                                            max_seqlen_k, pb.max_seqlen_bucket)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        out = pkg.attention_stored(t["kv_cache"], t["q"], meta)
+        return torch.cuda.max_memory_allocated() - before, out
+
+    own = t["cu_seqlens_k"].clone()
+    small = 4 << 20  # the output and the work list
+    size, want = run(256, own)
+    assert size < small
+    for given, cu_k in ((torch.tensor(200), own), (torch.tensor(200, device=dev), own), (None, t["cu_seqlens_q"]),
+                        (None, None)):
+        size, out = run(given, cu_k)
+        assert size < small and torch.equal(out, want)
+    for given in (None, 30000):  # the table, or the bound, leaves room for long items
+        size, out = run(given, own)
+        assert size > small
+        assert torch.equal(out, want)  # there are none: the kernel splits nothing
+
+
 def test_prefill_split_rows_without_keys_and_rows_past_the_bucket(pkg, dev):
     """Split launches: rows whose position precedes the first kv position,
     rows past max_seqlen_bucket and rows outside every sequence are zeros."""

@@ -4,6 +4,8 @@ checks raise the reference's ValueError messages (prefill_paged_attention.py:
 and CPU tensors are refused rather than computed on the host."""
 from __future__ import annotations
 
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -165,3 +167,15 @@ def test_other_quantized_page_dtypes_are_refused():
     with pytest.raises(ValueError, match="same dtype"):
         check_quantized_pages(torch.zeros(hkv, nb, bs, d, dtype=torch.int8),
                               torch.zeros(hkv, nb, bs, d, dtype=torch.uint8), sc, sc)
+
+
+@pytest.mark.parametrize("given,bound", [
+    (None, None), (4096, 4096), (np.int32(7), 7), (torch.tensor(33, dtype=torch.int32), 33),
+    (torch.tensor([33]), 33), (0, 0), (-5, 0),
+    # not a number on the host: accepted as before, and nothing is known
+    (torch.tensor([3, 4]), 0), (torch.tensor(3.5), 0), (torch.empty((), dtype=torch.int32, device="meta"), 0),
+    (np.array([3, 4]), 0), ("max", 0), (2.5, 0),
+])
+def test_prefill_metadata_kv_bound(given, bound):
+    got = sys.modules["vllm_jax_amd.attention"]._host_bound(given)
+    assert got == bound and type(got) is type(bound)

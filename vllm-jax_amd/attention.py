@@ -21,6 +21,7 @@ prefill or decode kernel.  Differences from the reference, all deliberate:
 """
 from __future__ import annotations
 
+import numbers
 import os
 from dataclasses import dataclass, field
 from typing import Optional, Tuple, Union
@@ -48,14 +49,22 @@ class DecodeAttentionMetadata:
 
 @dataclass
 class PrefillAttentionMetadata:
-    """qwen3.py:25-34 (``max_seqlen_bucket`` is static in the reference)."""
+    """qwen3.py:25-34 (``max_seqlen_bucket`` is static in the reference).
+
+    ``max_seqlen_k`` (unused by the reference's path) as an integer or a CPU
+    tensor of one tells the prefill the longest kv length where
+    ``block_tables`` is wider (launches of few items are then split by it, not
+    by the width); anything else, such as a device tensor, which is not read,
+    says that it is not known, ``None`` that the table is as wide as the
+    longest.  Where nothing is cached, ``cu_seqlens_k`` may be
+    ``cu_seqlens_q`` itself: the new tokens then bound the kv lengths."""
     input_positions: torch.Tensor
     slot_mapping: torch.Tensor
     block_tables: torch.Tensor
     cu_seqlens_q: torch.Tensor
     cu_seqlens_k: torch.Tensor
     max_seqlen_q: torch.Tensor
-    max_seqlen_k: torch.Tensor
+    max_seqlen_k: Union[torch.Tensor, int, None]
     max_seqlen_bucket: int = field(default=0)
 
 
@@ -261,6 +270,18 @@ def qwen3_attention_core(kv_cache: torch.Tensor, q: torch.Tensor, k: torch.Tenso
     return kv_cache, attention_stored(kv_cache, q_rot, metadata)
 
 
+def _host_bound(longest) -> Optional[int]:
+    """``PrefillAttentionMetadata.max_seqlen_k`` as the prefill takes it, without
+    reading device memory; 0 for anything that is not a number on the host."""
+    if longest is None:
+        return None
+    if isinstance(longest, torch.Tensor):
+        if longest.device.type != "cpu" or longest.numel() != 1 or longest.is_floating_point():
+            return 0
+        longest = longest.item()
+    return max(0, int(longest)) if isinstance(longest, numbers.Integral) else 0
+
+
 def attention_stored(kv_cache: torch.Tensor, q: torch.Tensor, metadata: AttentionMetadata) -> torch.Tensor:
     """The attention part of qwen3.py:175-218 for K/V already in the pool."""
     if not (USE_PREFILL_PAGED_ATTENTION_KERNEL and USE_DECODE_PAGED_ATTENTION_KERNEL):
@@ -279,7 +300,8 @@ def attention_stored(kv_cache: torch.Tensor, q: torch.Tensor, metadata: Attentio
             decode_scale=1.0 / bf16_round(float(head_dim) ** 0.5))
     elif isinstance(metadata, PrefillAttentionMetadata):
         tables = (metadata.block_tables, metadata.cu_seqlens_q)
-        kw = dict(max_seqlen_bucket=metadata.max_seqlen_bucket, cu_seqlens_k=metadata.cu_seqlens_k)
+        kw = dict(max_seqlen_bucket=metadata.max_seqlen_bucket, cu_seqlens_k=metadata.cu_seqlens_k,
+                  max_seqlen_k=_host_bound(metadata.max_seqlen_k))
         if pool:
             outputs = prefill_pool(q, kv_cache, *tables, metadata.input_positions, **kw)
         else:

@@ -51,6 +51,7 @@ def prefill_paged_attention(
         scale: float | None = None,
         out: torch.Tensor | None = None,
         workspace: torch.Tensor | None = None,
+        max_seqlen_k: int | None = None,
 ) -> torch.Tensor:
     """Paged prefill attention; returns ``[T, H, d]`` bf16.
 
@@ -66,7 +67,11 @@ def prefill_paged_attention(
         also splits them over their kv range) and, for
         quantized pages (float8 e4m3fn codes, or int8 / uint8 integers, with
         float32 ``[Hkv, NB, BS]`` per-token scales), the pages widened to bf16 ahead of it
-        (``pa_prefill_fp8_workspace_size``); allocated when absent or too small.
+        (``pa_prefill_fp8_workspace_size``); allocated when absent or too small;
+      * ``max_seqlen_k`` -- a bound on the kv lengths (0: none is known), where
+        ``block_tables`` is wider than the longest of them: launches are split
+        by the bound instead of the table's width.  It changes no result but
+        the last bits of a launch that it keeps whole.
     """
     del slot_mapping, block_m, pages_per_compute_block, k_splits, num_warps, num_stages
     del interpret, debug, mask_value
@@ -89,12 +94,12 @@ def prefill_paged_attention(
                                            k_scales_pages.stride(1), k_scales_pages.stride(0))
     return _prefill(q, (num_kv_heads, num_pages, page_size, head_dim), (k_pages.data_ptr(), v_pages.data_ptr()),
                     pages_strides(k_pages), code_type, scales, block_tables, cu_seqlens, input_positions,
-                    max_seqlen_bucket, attn_logits_soft_cap, cu_seqlens_k, scale, out, workspace)
+                    max_seqlen_bucket, attn_logits_soft_cap, cu_seqlens_k, scale, out, workspace, max_seqlen_k)
 
 
 def prefill_pool(q: torch.Tensor, kv_cache: torch.Tensor, block_tables: torch.Tensor, cu_seqlens: torch.Tensor,
                  input_positions: torch.Tensor, *, max_seqlen_bucket: int,
-                 cu_seqlens_k: torch.Tensor | None = None) -> torch.Tensor:
+                 cu_seqlens_k: torch.Tensor | None = None, max_seqlen_k: int | None = None) -> torch.Tensor:
     """:func:`prefill_paged_attention` over the halves of the engine's bf16
     pool ``[2, NB, BS, Hkv, d]``, without making the page views."""
     require_device("kv_cache", kv_cache)
@@ -103,7 +108,8 @@ def prefill_pool(q: torch.Tensor, kv_cache: torch.Tensor, block_tables: torch.Te
     _check_shapes(q, (num_kv_heads, num_pages, page_size, head_dim), block_tables, cu_seqlens, cu_seqlens_k)
     _, ps, ss, hs, _ = kv_cache.stride()
     return _prefill(q, (num_kv_heads, num_pages, page_size, head_dim), pool_pointers(kv_cache), (ps, ss, hs), None, (),
-                    block_tables, cu_seqlens, input_positions, max_seqlen_bucket, None, cu_seqlens_k, None, None, None)
+                    block_tables, cu_seqlens, input_positions, max_seqlen_bucket, None, cu_seqlens_k, None, None, None,
+                    max_seqlen_k)
 
 
 def _check_shapes(q, pages, block_tables, cu_seqlens, cu_seqlens_k):
@@ -127,7 +133,7 @@ def _check_shapes(q, pages, block_tables, cu_seqlens, cu_seqlens_k):
 
 
 def _prefill(q, pages, pointers, strides, code_type, scales, block_tables, cu_seqlens, input_positions,
-             max_seqlen_bucket, attn_logits_soft_cap, cu_seqlens_k, scale, out, workspace):
+             max_seqlen_bucket, attn_logits_soft_cap, cu_seqlens_k, scale, out, workspace, max_seqlen_k):
     """The launch for checked pages: ``pages`` = (Hkv, NB, BS, d), ``pointers``
     and element ``strides`` (page, slot, head) of K and V, ``scales`` =
     pointers and (page, head) strides of quantized pages' scales."""
@@ -160,15 +166,23 @@ def _prefill(q, pages, pointers, strides, code_type, scales, block_tables, cu_se
     if quantized:
         extra = int(lib.pa_prefill_fp8_workspace_size(batch, pages_per_sequence, page_size, num_kv_heads, head_dim,
                                                       int(max_seqlen_bucket), num_heads)) - need
-    if workspace is None or workspace.numel() * workspace.element_size() < need + extra:
-        # our own: with room for the parts of a launch that splits its items
+    given = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    if given < need + extra or max_seqlen_k is not None:
+        pages = pages_per_sequence
+        if max_seqlen_k is not None:
+            pages = min(pages, -(-max(0, int(max_seqlen_k)) // page_size))
         cached = cuk is not None and cuk.data_ptr() != cu.data_ptr()
-        if lib.pa_prefill_route(batch, total_tokens, int(max_seqlen_bucket), num_heads, num_kv_heads, head_dim,
-                                pages_per_sequence, page_size, cached) == _ROUTE_SPLIT:
-            need = int(lib.pa_prefill_split_workspace_size(batch, int(max_seqlen_bucket), num_heads, num_kv_heads,
-                                                           head_dim, pages_per_sequence, page_size))
-        workspace = torch.empty(max(need + extra, 1), dtype=torch.uint8, device=q.device)
-    ws_bytes = workspace.numel() * workspace.element_size()
+        split = lib.pa_prefill_route(batch, total_tokens, int(max_seqlen_bucket), num_heads, num_kv_heads, head_dim,
+                                     pages, page_size, cached) == _ROUTE_SPLIT
+        if given < need + extra:
+            # our own: with room for the parts of a launch that splits its items
+            if split:
+                need = int(lib.pa_prefill_split_workspace_size(batch, int(max_seqlen_bucket), num_heads, num_kv_heads,
+                                                               head_dim, pages_per_sequence, page_size))
+            given = max(need + extra, 1)
+            workspace = torch.empty(given, dtype=torch.uint8, device=q.device)
+        elif not split:
+            given = need + extra  # no room for parts
     if quantized:
         _lib.call(
             "pa_prefill_quant", code_type,
@@ -182,7 +196,7 @@ def _prefill(q, pages, pointers, strides, code_type, scales, block_tables, cu_se
             num_heads, num_kv_heads, head_dim,
             float(scale), soft_cap,
             out.data_ptr(), out.stride(0), out.stride(1),
-            workspace.data_ptr(), ws_bytes,
+            workspace.data_ptr(), given,
             stream_handle(q))
         return out
     _lib.call(
@@ -196,6 +210,6 @@ def _prefill(q, pages, pointers, strides, code_type, scales, block_tables, cu_se
         num_heads, num_kv_heads, head_dim,
         float(scale), soft_cap,
         out.data_ptr(), out.stride(0), out.stride(1),
-        workspace.data_ptr(), ws_bytes,
+        workspace.data_ptr(), given,
         stream_handle(q))
     return out
