@@ -169,8 +169,14 @@ size_t pa_decode_noalloc_max_workspace(void);
  * q/out: [num_tokens, H, d] with (tok, head) strides.
  * workspace (256-byte aligned, pa_prefill_workspace_size bytes, or NULL)
  * holds a work list that orders the (q tile, sequence, kv head) items by
- * their kv length, longest first; it changes no result.  Without it (or for
- * batch > 2048) items run from the last q tile down.
+ * their kv length, longest first; the list changes no result.  Without it (or
+ * for batch > 2048) items run from the last q tile down.  A workspace of
+ * pa_prefill_split_workspace_size bytes or more, given for whatever reason,
+ * lets a launch of few, long items split them (PA_PREFILL_SPLIT): P is then
+ * rounded relative to each part's own reference max and the part length
+ * follows the whole batch, so that a row's last bits differ from those of the
+ * unsplit launch and depend on the other sequences' lengths.  Give the list's
+ * size where results must not.
  */
 int pa_prefill(const uint16_t* q, int64_t q_tok_stride, int64_t q_head_stride,
                const uint16_t* k_cache, const uint16_t* v_cache,
@@ -190,7 +196,8 @@ int pa_prefill(const uint16_t* q, int64_t q_tok_stride, int64_t q_head_stride,
  * launches: pa_prefill_workspace_size).  A workspace between the two sizes
  * runs unsplit.  pa_prefill_quant and pa_prefill_fp8 split when theirs is
  * larger than pa_prefill_fp8_workspace_size by this minus
- * pa_prefill_workspace_size.  0 for bad sizes; no counterpart in the
+ * pa_prefill_workspace_size.  The parts change the last bits of the results
+ * (pa_prefill).  0 for bad sizes; no counterpart in the
  * reference, whose prefill grid is fixed. */
 size_t pa_prefill_split_workspace_size(int32_t batch, int32_t max_seqlen_q, int32_t num_heads, int32_t num_kv_heads,
                                        int32_t head_dim, int32_t pages_per_seq, int32_t page_size);

@@ -64,7 +64,8 @@ def prefill_paged_attention(
       * ``workspace`` -- device bytes for the work list that orders the
         kernel's items by kv length (``pa_prefill_workspace_size``; with
         ``pa_prefill_split_workspace_size`` bytes a launch of few, long items
-        also splits them over their kv range) and, for
+        also splits them over their kv range, which changes the last bits of
+        its results by the batch's lengths) and, for
         quantized pages (float8 e4m3fn codes, or int8 / uint8 integers, with
         float32 ``[Hkv, NB, BS]`` per-token scales), the pages widened to bf16 ahead of it
         (``pa_prefill_fp8_workspace_size``); allocated when absent or too small;
