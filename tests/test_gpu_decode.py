@@ -209,6 +209,10 @@ def test_decode_work_list_many_q_heads_per_kv_head(pkg, dev):
     ([600, 2300], 32, 8, 24, 128),                     # pages that are not whole steps
     (list(range(1, 256)) + [480], 8, 4, 16, 32),       # 256 sequences, several rounds of single parts
     ([2048 * 3], 24, 2, 64, 96),                       # G = 12
+    ([11400] * 3, 32, 8, 64, 256),                     # equal lengths, a few parts too many: a fifteenth longer
+    ([2100] * 17, 16, 8, 16, 256),                     # the same, a quarter longer
+    ([3000] * 100 + [7], 4, 1, 64, 64),                # the same over more than 64 sequences
+    ([2600, 1900] * 20, 16, 8, 32, 128),               # too many either way
 ])
 def test_decode_parts_cut_on_the_device(pkg, dev, lens, h, hkv, bs, width):
     """Launches without a work list cut ragged sequences into equal parts by

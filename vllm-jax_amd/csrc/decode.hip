@@ -71,23 +71,31 @@ __device__ __forceinline__ int ceil_div_small(int x, int d) {
 }
 
 // The work item of workgroup blockIdx.x in a launch that cuts its sequences
-// on the device: every workgroup sums the lengths (one thread per sequence),
+// on the device: every workgroup sums the lengths (one thread per sequence; up
+// to 64 sequences each wave by itself, without a barrier),
 // takes an even share of a resident workgroup as the part length L (at least
 // kDecodeMinChunk, at most p.balance_cap tokens), cuts each sequence into
 // equal parts of at most L and ranks the parts, those longer than L / 2
 // first, so that a ragged batch neither waits for its longest chunk nor
-// starts one last.  If that takes more partials than the workspace holds, L
-// is the cap, whose parts it is sized for.  XCD x = bid % 8 takes ranks x,
+// starts one last.  Where that makes a few parts more than are resident at
+// once, which equal sequences would wait a whole second part for, L grows by a
+// fifteenth or a quarter if the parts then fit.  If it takes more partials than
+// the workspace holds, L is the cap, whose parts it is sized for.  XCD x = bid % 8 takes ranks x,
 // x + 8, ..., all kv heads of a rank in a row (as with the work list).  False:
 // nothing to do.
-// Against fixed chunks of 2048 tokens (1024 over 16-token pages) in sequence
-// order, whole calls in one process, Qwen3-8B heads: 16 sequences of 500 to
-// 16000 tokens 144.3 -> 121 us, 48 of 200 to 4000 98.0 -> 84, 24 of 200 to
-// 8000 over 16-token pages 107 -> 85, 128 of 100 to 2000 110.7 -> 98.
+// Against fixed chunks (2048 tokens, 1024 over 16-token pages, half or a quarter
+// on small launches) in sequence order, whole calls, 32 / 8 heads: 16 sequences
+// of 500 to 16000 tokens 144 -> 121 us, 48 of 200 to 4000 95.1 -> 83.0, 128 of
+// 100 to 2000 108.3 -> 100.3, 24 of 200 to 8000 over 16-token pages (16 / 8
+// heads) 105 -> 83.3.  Equal lengths: 3 x 30000 72.2 -> 70.0 (81.6 before L
+// grew), 10 x 6000 48.9 -> 48.9 (55.7), 16 x 8192 95.2 -> 95.0; the cut itself
+// shows at 2 x 16384, 29.3 -> 30.0, and 64 x 2048, 92.6 -> 93.7.
 __device__ __forceinline__ bool decode_balance(const DecodeParams& p, DecodeWork& w) {
   __shared__ uint32_t s_sum[kDecodeWaves], s_cls[kDecodeWaves], s_slots[kDecodeWaves];
-  __shared__ int32_t s_work[7];
+  __shared__ int32_t s_work[6];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool alone = p.batch <= 64;  // uniform: each wave counts all sequences by itself
+  const int seq = alone ? lane : tid;
   const int hkv = p.num_kv_heads;
   const int vheads = hkv * p.hblocks;
   const int k = blockIdx.x >> 3;
@@ -95,17 +103,31 @@ __device__ __forceinline__ bool decode_balance(const DecodeParams& p, DecodeWork
   const int mine = 8 * kr + (blockIdx.x & 7);
   w.vh = k - kr * vheads;
   // launches without a work list span fewer than 2^23 tokens over all table rows
-  const int len = tid < p.batch ? max(0, min(p.lengths[tid], p.pages_per_seq * p.page_size)) : 0;
-  const uint32_t sum = wave_scan((uint32_t)len);
-  if (lane == 63) s_sum[wave] = sum;
+  const int len = seq < p.batch ? max(0, min(p.lengths[seq], p.pages_per_seq * p.page_size)) : 0;
   if (tid == 0) s_work[0] = -1;
-  __syncthreads();
-  const uint32_t total = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+  // the sum over all sequences
+  auto sum_all = [&](uint32_t v) __attribute__((always_inline)) -> uint32_t {
+    const uint32_t upto = wave_scan(v);
+    if (alone) return (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
+    __syncthreads();  // the last sum has been read
+    if (lane == 63) s_sum[wave] = upto;
+    __syncthreads();
+    return s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+  };
+  const uint32_t total = sum_all((uint32_t)len);
   const int align = balance_align(p.page_size);
   const uint64_t share = ((uint64_t)total * (uint32_t)vheads + kBalanceSlots - 1) / kBalanceSlots;
   int most = share >= (uint64_t)p.balance_cap
                  ? p.balance_cap
                  : min(p.balance_cap, max(kDecodeMinChunk, ((int)share + align - 1) & -align));
+  // whether the parts of at most `part` tokens are resident at once
+  auto fits = [&](int part) __attribute__((always_inline)) {
+    return sum_all((uint32_t)ceil_div_small(len, part)) * (uint32_t)vheads <= (uint32_t)kBalanceSlots;
+  };
+  if (p.batch * vheads < kBalanceSlots && !fits(most)) {  // uniform
+    const int fourth = (most + most / 4 + align - 1) & -align, little = (most + most / 15 + align - 1) & -align;
+    if (fourth <= p.balance_cap && fits(fourth)) most = fits(little) ? little : fourth;
+  }
   int parts, size, start, slot;
   while (true) {
     size = (ceil_div_small(len, max(1, ceil_div_small(len, most))) + align - 1) & -align;
@@ -115,48 +137,58 @@ __device__ __forceinline__ bool decode_balance(const DecodeParams& p, DecodeWork
     const uint32_t mine_cls = (uint32_t)parts << (small ? 16 : 0);
     uint32_t run = wave_scan(mine_cls);
     slot = (int)wave_scan(parts > 1 ? (uint32_t)parts : 0u);
-    if (lane == 63) {
-      s_cls[wave] = run;
-      s_slots[wave] = (uint32_t)slot;
-    }
-    __syncthreads();
-    uint32_t all = 0;
-    int slots = 0;
+    uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)run, 63);
+    int slots = __builtin_amdgcn_readlane(slot, 63);
+    if (!alone) {
+      if (lane == 63) {
+        s_cls[wave] = run;
+        s_slots[wave] = (uint32_t)slot;
+      }
+      __syncthreads();
+      all = 0;
+      slots = 0;
 #pragma unroll
-    for (int i = 0; i < kDecodeWaves; ++i) {
-      run += i < wave ? s_cls[i] : 0;
-      slot += i < wave ? (int)s_slots[i] : 0;
-      all += s_cls[i];
-      slots += (int)s_slots[i];
+      for (int i = 0; i < kDecodeWaves; ++i) {
+        run += i < wave ? s_cls[i] : 0;
+        slot += i < wave ? (int)s_slots[i] : 0;
+        all += s_cls[i];
+        slots += (int)s_slots[i];
+      }
     }
     start = (small ? (int)(run >> 16) + (int)(all & 0xffff) : (int)(run & 0xffff)) - parts;
     slot -= parts > 1 ? parts : 0;
     if (slots <= p.balance_slots || most == p.balance_cap) break;  // uniform
     most = p.balance_cap;
-    __syncthreads();
-  }
-  if (mine >= start && mine < start + parts) {
-    const int i = mine - start;
-    s_work[0] = tid;
-    s_work[1] = i * size;
-    s_work[2] = min(i * size + size, len);
-    s_work[3] = len;
-    s_work[4] = parts;
-    s_work[5] = slot;
-    s_work[6] = i;
+    if (!alone) __syncthreads();
   }
   if (blockIdx.x == 0 && tid < p.batch) p.balance[tid] = (int32_t)((uint32_t)slot << 16 | (uint32_t)parts);
-  __syncthreads();
-  auto work = [&](int i) { return __builtin_amdgcn_readfirstlane(s_work[i]); };
-  w.b = work(0);
-  if (w.b < 0) return false;
-  w.t_begin = work(1);
-  w.t_end = work(2);
-  w.len = work(3);
-  const int n = work(4);
-  w.single = n == 1;
+  // the owner's values of this workgroup's part `i`
+  const int i = mine - start;
+  const bool own = i >= 0 && i < parts;
+  int v[6] = {seq, i, size, len, parts, slot};
+  if (alone) {
+    const uint64_t owner = __ballot(own);
+    if (!owner) return false;
+    const int l = __ffsll((unsigned long long)owner) - 1;
+#pragma unroll
+    for (int e = 0; e < 6; ++e) v[e] = __builtin_amdgcn_readlane(v[e], l);
+  } else {
+    if (own) {
+#pragma unroll
+      for (int e = 0; e < 6; ++e) s_work[e] = v[e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 6; ++e) v[e] = __builtin_amdgcn_readfirstlane(s_work[e]);
+    if (v[0] < 0) return false;
+  }
+  w.b = v[0];
+  w.t_begin = v[1] * v[2];
+  w.t_end = min(w.t_begin + v[2], v[3]);
+  w.len = v[3];
+  w.single = v[4] == 1;
   // a sequence's partials: its parts within each kv head
-  w.part = (int64_t)work(5) * hkv + (int64_t)(w.vh / p.hblocks) * n + work(6);
+  w.part = (int64_t)v[5] * hkv + (int64_t)(w.vh / p.hblocks) * v[4] + v[1];
   return true;
 }
 
