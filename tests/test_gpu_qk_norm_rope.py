@@ -182,7 +182,7 @@ def test_qk_norm_rope_store_qwen3_32b_long_workload(pkg, dev):
     _close(u16(flat_k[slots[idx]]), kc_want.reshape(sel.size, hkv, d))
 
 
-@pytest.mark.parametrize("h,hkv", [(16, 8), (32, 8), (64, 8), (5, 1)])
+@pytest.mark.parametrize("h,hkv", [(16, 8), (32, 8), (64, 8), (5, 1), (48, 8), (49, 8), (128, 8), (4, 2)])
 def test_qk_norm_rope_store_few_tokens_bit_identical(pkg, dev, h, hkv):
     """Launches of few tokens deal a token's rows to several waves: each
     token's outputs equal, bit for bit, those of a launch of 4 200 tokens

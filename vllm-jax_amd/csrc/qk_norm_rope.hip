@@ -92,6 +92,7 @@ qk_norm_rope_store_kernel(RopeParams p) {
   const int nq = p.num_heads;
   const int nqk = p.num_heads + p.num_kv_heads;
   const int rows = nqk + p.num_kv_heads;
+  if (first >= rows) return;  // no batch left for this wave
 
   // row r of this token: q heads, then k heads, then v heads
   auto row_src = [&](int r) -> const uint16_t* {
@@ -188,19 +189,21 @@ qk_norm_rope_store_kernel(RopeParams p) {
 
 // log2 of the waves a token's rows are dealt to.  With few tokens the launch
 // is a serial chain, not a stream: one wave walks 32 to 80 rows in batches of
-// 8 or 16, each batch waiting for its loads.  Dealing the batches to 2, 4 or 8
+// 8 or 16, each batch waiting for its loads.  Dealing the `batches` to 2, 4 or 8
 // waves (each evaluates the rotation again) shortens the chain while the chip
-// still has room for them: up to kRopeWaves waves, and no more parts than
-// there are 8-row batches.  Measured over back-to-back launches, one wave a
+// still has room for them: up to kRopeWaves waves, and no more than leave each
+// at most one batch (a power of two, so some of the last may have none; they
+// return at once).
+// Measured over back-to-back launches, one wave a
 // token -> this rule: 32 / 8 heads 4 tokens 9.0 -> 4.7 us, 256 10.8 -> 4.9,
 // 1000 11.1 -> 8.2, 2000 15.5 -> 13.0; 64 / 8 heads 4 tokens 13.4 -> 5.2,
 // 1000 17.7 -> 11.9.  Past the limit the extra waves only repeat the rotation
 // (16 / 8 heads, 4096 tokens: 16.0 us with one, 17.4 with two, 18.7 with
 // four).
 constexpr int64_t kRopeWaves = 4096;
-static int rope_part_bits(int64_t tokens, int64_t rows) {
+static int rope_part_bits(int64_t tokens, int64_t batches) {
   int bits = 0;
-  while (bits < 3 && (tokens << (bits + 1)) <= kRopeWaves && (8 << bits) < rows) ++bits;
+  while (bits < 3 && (tokens << (bits + 1)) <= kRopeWaves && (1 << bits) < batches) ++bits;
   return bits;
 }
 
@@ -309,9 +312,11 @@ extern "C" int pa_qk_norm_rope_store(const uint16_t* q, int64_t q_tok_stride, in
   prm.scale_pos = rope_scaling_factor != 1.f;
   prm.pos_div = rope_scaling_factor;
   rope_inv_freq(rope_theta, prm.inv_freq);
-  prm.part_bits = rope_part_bits(num_tokens, (int64_t)num_heads + 2 * (int64_t)num_kv_heads);
+  const int64_t rows = (int64_t)num_heads + 2 * (int64_t)num_kv_heads;
+  const bool wide = rows >= 64;  // batches of 16 rows, else of 8
+  prm.part_bits = rope_part_bits(num_tokens, wide ? (rows + 15) / 16 : (rows + 7) / 8);
   const int64_t blocks = (((int64_t)num_tokens << prm.part_bits) + 3) / 4;
-  if (num_heads + 2 * num_kv_heads >= 64)
+  if (wide)
     qk_norm_rope_store_kernel<4, true><<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(prm);
   else
     qk_norm_rope_store_kernel<2, false><<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(prm);
