@@ -208,7 +208,7 @@ def test_decode_work_list_many_q_heads_per_kv_head(pkg, dev):
     ([1024, 1023, 3000], 32, 8, 16, 256),              # 16-token pages: parts of up to 1024 tokens
     ([600, 2300], 32, 8, 24, 128),                     # pages that are not whole steps
     (list(range(1, 256)) + [480], 8, 4, 16, 32),       # 256 sequences, several rounds of single parts
-    ([2048 * 3], 24, 2, 64, 96),                       # G = 12
+    ([2048 * 3, 700, 1500], 24, 2, 64, 96),            # G = 12
     ([11400] * 3, 32, 8, 64, 256),                     # equal lengths, a few parts too many: a fifteenth longer
     ([2100] * 17, 16, 8, 16, 256),                     # the same, a quarter longer
     ([3000] * 100 + [7], 4, 1, 64, 64),                # the same over more than 64 sequences
@@ -217,6 +217,7 @@ def test_decode_work_list_many_q_heads_per_kv_head(pkg, dev):
 def test_decode_parts_cut_on_the_device(pkg, dev, lens, h, hkv, bs, width):
     """Launches without a work list cut ragged sequences into equal parts by
     an even share of the batch's tokens: every sequence against the oracle."""
+    assert 1 < len(lens) <= 256  # one sequence alone keeps the fixed chunks
     db = wl.make_decode(lens, num_heads=h, num_kv_heads=hkv, page_size=bs, rng=np.random.default_rng(len(lens)),
                         table_width=width)
     out, _ = _run_and_check(pkg, dev, db, seed=5)

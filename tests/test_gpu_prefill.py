@@ -433,8 +433,8 @@ def test_prefill_page_sizes_bit_identical(pkg, dev, prefix):
     ([2000, 100], [65, 64], 64, 2, 24, None),             # G = 32, per-lane paging
     ([3000], [1], 8, 1, 64, None),                        # one row, one kv head: 8 q rows, many parts
     ([0], [1999], 16, 8, 16, None),                       # a fresh prompt: only its long items split
-    ([1600, 1, 0, 5], [0, 3, 128, 129], 12, 3, 32, None),  # a sequence without rows, 3 kv heads
-    ([1600, 2500, 5, 900], [70, 0, 129, 100], 12, 3, 32, None),  # real parts at 3 kv heads, whose share does not divide
+    ([1600, 1, 0, 5], [0, 3, 128, 129], 12, 3, 32, None),  # the long sequence has no rows: nothing is split
+    ([1600, 2500, 5, 900], [70, 0, 129, 100], 12, 3, 32, None),  # parts at 3 kv heads, whose share does not divide
     ([0, 3000, 0], [300, 40, 500], 16, 1, 64, None),       # one kv head, 16-token tiles: 96 pairs
     ([0], [2500], 16, 1, 64, None),                        # as many pairs as there can be
 ])
@@ -459,6 +459,9 @@ def test_prefill_split_items(pkg, dev, prefix, new, h, hkv, bs, cap):
     kw = dict(max_seqlen_bucket=pb.max_seqlen_bucket, cu_seqlens_k=t["cu_seqlens_k"], attn_logits_soft_cap=cap)
     one = pkg.prefill_paged_attention(*args, workspace=torch.empty(plan, dtype=torch.uint8, device=dev), **kw)
     assert np.abs(got - ora.bf16_to_f32(u16(one))).max() <= TOL
+    # parts round P by references of their own: some of the last bits differ
+    # exactly when an item was split
+    assert np.array_equal(got, ora.bf16_to_f32(u16(one))) == (max(p + n for p, n in zip(prefix, new) if n) < 1536)
     # a workspace full of NaNs (stale partials) changes nothing
     ws = torch.full((split,), 255, dtype=torch.uint8, device=dev)
     two = pkg.prefill_paged_attention(*args, workspace=ws, **kw)
