@@ -213,6 +213,9 @@ def test_decode_work_list_many_q_heads_per_kv_head(pkg, dev):
     ([2100] * 17, 16, 8, 16, 256),                     # the same, a quarter longer
     ([3000] * 100 + [7], 4, 1, 64, 64),                # the same over more than 64 sequences
     ([2600, 1900] * 20, 16, 8, 32, 128),               # too many either way
+    ([2000] * 32, 16, 4, 64, 32),                      # more parts than slots: the fixed chunk of 1024
+    (list(range(100, 2020, 30)), 32, 8, 256, 8),       # one chunk a sequence: longer parts until the slots do
+    (list(range(60, 2040, 22)), 16, 4, 64, 32),        # the same over more than 64 sequences
 ])
 def test_decode_parts_cut_on_the_device(pkg, dev, lens, h, hkv, bs, width):
     """Launches without a work list cut ragged sequences into equal parts by

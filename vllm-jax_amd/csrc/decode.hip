@@ -80,7 +80,11 @@ __device__ __forceinline__ int ceil_div_small(int x, int d) {
 // starts one last.  Where that makes a few parts more than are resident at
 // once, which equal sequences would wait a whole second part for, L grows by a
 // fifteenth or a quarter if the parts then fit.  If it takes more partials than
-// the workspace holds, L is the cap, whose parts it is sized for.  XCD x = bid % 8 takes ranks x,
+// the workspace holds, L is the fixed chunk, whose parts it is sized for (a
+// length between, a quarter longer at a time, took 36 us where the chunk takes
+// 28: 64 sequences of 500 to 8000 tokens, 8 / 1 heads; only where one chunk holds
+// any sequence is that length tried: 64 of 100 to 2000, 32 / 8 heads, 67.5 ->
+// 64).  XCD x = bid % 8 takes ranks x,
 // x + 8, ..., all kv heads of a rank in a row (as with the work list).  False:
 // nothing to do.
 // Against fixed chunks (2048 tokens, 1024 over 16-token pages, half or a quarter
@@ -157,8 +161,9 @@ __device__ __forceinline__ bool decode_balance(const DecodeParams& p, DecodeWork
     }
     start = (small ? (int)(run >> 16) + (int)(all & 0xffff) : (int)(run & 0xffff)) - parts;
     slot -= parts > 1 ? parts : 0;
-    if (slots <= p.balance_slots || most == p.balance_cap) break;  // uniform
-    most = p.balance_cap;
+    if (slots <= p.balance_slots || most >= p.chunk) break;  // uniform
+    // (strictly longer each time, up to the chunk)
+    most = p.n_chunks == 1 ? min(p.chunk, (most + most / 4 + align - 1) & -align) : p.chunk;
     if (!alone) __syncthreads();
   }
   if (blockIdx.x == 0 && tid < p.batch) p.balance[tid] = (int32_t)((uint32_t)slot << 16 | (uint32_t)parts);
@@ -480,15 +485,20 @@ extern "C" size_t pa_decode_workspace_size(int32_t batch, int32_t num_heads, int
 }
 
 // Whether a launch of `p` (with `fits`: decode_split_kernel's, without a work
-// list, and with pages) cuts its sequences on the device: not one sequence
-// alone (its chunks are equal; the cut costs about 1 us), and not when every
-// sequence is one short part and all of them are resident at once, where
-// neither the cut nor the order matters.  The token bound is decode_balance's
-// (any launch without a work list meets it at 8 kv heads and more).
+// list, and with pages) cuts its sequences on the device.  Not one sequence
+// alone, whose chunks are equal.  Where a fixed chunk holds the longest sequence
+// the workspace has one partial per sequence, and the cut, about 1 us (1.5 of
+// more than 64 sequences), gains by the order of the parts and by cutting a few
+// of them: ragged sequences of up to 2000 tokens 5 to 12 % from about 256
+// workgroups on, and nothing below that or at 1024 tokens (70 of 1 to 512
+// tokens, 32 / 8 heads, 22.1 us without the cut and 26.7 with it; 238 of 274,
+// 59.1 and 63.0; 70 of 1500 at 8 / 1 heads 20.8 and 22.4).  The token bound is
+// decode_balance's (any launch without a work list meets it at 8 kv heads and
+// more).
 static bool decode_balanced(const DecodeParams& p, bool fits, int span, int64_t vheads) {
   const int64_t tokens = (int64_t)p.pages_per_seq * p.page_size;
   return fits && span <= 64 && p.batch > 1 && p.batch <= kBalanceMaxBatch && tokens * p.batch < (1 << 23) &&
-         (tokens > kDecodeMinChunk || p.batch * vheads > kBalanceSlots);
+         (p.n_chunks > 1 || (tokens > 1024 && p.batch * vheads > kBalanceSlots / 2));
 }
 
 // Shared argument checks and launch of pa_decode / pa_decode_fp8.  `prm`
@@ -625,10 +635,8 @@ static int decode_common(const char* name, DecodeParams& prm, bool fp8, const ui
     prm.balance = plan;  // one int per sequence, in the work list's place
     prm.balance_slots = (int32_t)pairs;
     prm.balance_cap = decode_chunk_tokens(page_size);
-    // parts of at least an even share, or of the cap (decode_balance)
-    const int64_t cap_parts =
-        (int64_t)batch * (((int64_t)pages_per_seq * page_size + prm.balance_cap - 1) / prm.balance_cap);
-    blocks = (std::max<int64_t>(kBalanceSlots / vheads + batch, cap_parts) + 7) / 8 * 8 * vheads;
+    // parts of at least an even share, or of the fixed chunk (decode_balance)
+    blocks = (std::max<int64_t>(kBalanceSlots / vheads + batch, pairs) + 7) / 8 * 8 * vheads;
   }
   if (planned) {
     decode_plan_kernel<<<dim3(1), dim3(kPlanThreads), 0, s>>>(prm, plan);
