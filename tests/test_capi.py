@@ -361,6 +361,9 @@ def test_prefill_split_workspace_size():
     # more than a round, but the longest item decides
     ([1500], 0, 32, 8, False), ([2000], 0, 32, 8, False), ([700] * 2, 0, 32, 8, False),
     ([4000], 0, 16, 8, False), ([1400] * 2, 0, 16, 8, False), ([4000], 0, 16, 1, False),
+    # ragged: the longest decides, not the number of items
+    ([914, 1336, 439, 206], 0, 16, 8, False), ([2693, 1426, 1523, 2000], 0, 8, 8, False),
+    ([500, 100, 324, 225], 0, 32, 8, False),
     # several rounds
     ([3000], 0, 32, 8, True), ([511] * 4, 0, 32, 8, True), ([200] * 5, 0, 32, 8, True),
     ([1000] * 2, 4000, 32, 8, True), ([300] * 4, 4000, 32, 8, True), ([128] * 16, 0, 32, 8, True),

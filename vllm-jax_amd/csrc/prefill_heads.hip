@@ -63,11 +63,11 @@ int paging_of(const PrefillParams& p) {
 
 }  // namespace
 
-// Items of `tokens`-token tiles a launch can have at most: a sequence of n
-// tokens has ceil(n / tokens) of them per kv head.
-static int64_t items_of(const PrefillParams& p, int64_t tokens) {
-  const int64_t grid = p.batch * ((p.max_seqlen_q + tokens - 1) / tokens);
-  return std::min(grid, (p.num_tokens + p.batch * (tokens - 1)) / tokens) * p.num_kv_heads;
+// Items of `tokens`-token tiles a launch has, about: a sequence of n tokens has
+// ceil(n / tokens) of them per kv head, half a tile more than its tokens fill.
+static double items_of(const PrefillParams& p, int64_t tokens) {
+  const double grid = (double)p.batch * ((p.max_seqlen_q + tokens - 1) / tokens);
+  return std::min(grid, (double)p.num_tokens / tokens + .5 * p.batch) * p.num_kv_heads;
 }
 
 // Whether a launch at head size 256 is faster tiled than in the generic
@@ -78,11 +78,13 @@ static int64_t items_of(const PrefillParams& p, int64_t tokens) {
 // the tiled kernel's other waves skip their work; a launch of several rounds
 // is tiled, and in between the two estimates decide: the longest item, or all
 // of them over the CUs.  kv lengths are on the device.  The longest is taken
-// from the table's width, or, where cu_seqlens_k says that nothing is cached
+// from the table's width (its last page half full), or, where cu_seqlens_k says that nothing is cached
 // (and in a mixed launch, whose table is as wide as its decode sequences),
-// from max_seqlen_q; the others are taken to be as long.
-// Generic -> tiled, 32 / 8 heads unless said, us (both kernels measured at 400
-// shapes; this rule takes the slower one by 4 % at most, in 4 of them): generic
+// from max_seqlen_q; the others are taken to be as long, or, up to max_seqlen_q,
+// to have nothing cached.
+// Generic -> tiled, 32 / 8 heads unless said, us (both kernels timed at 740
+// shapes, 400 of them with the soft cap as well; this rule is never more than
+// 2 % behind the generic one): generic
 // 3 x 299 tokens 28.0 -> 31.5, 1 x 2000 118 -> 131, 1 x 1000 behind 4000
 // cached 237 -> 302, 16 / 8 heads 1 x 4000 211 -> 246; tiled 4 x 511 50.3 ->
 // 46.6, 1 x 3000 258 -> 190, 4 x 300 behind 4000 384 -> 265, 8 / 8 heads 8 x 64
@@ -93,17 +95,18 @@ static bool tiled_256_pays(const PrefillParams& p) {
   const double span = (double)p.pages_per_seq * p.page_size;
   const int64_t seq_rows = (int64_t)p.max_seqlen_q * p.group;
   if (seq_rows > 32 && seq_rows <= rows) return true;
-  if (seq_rows > 32 && seq_rows <= kRows && mean <= 64 && span <= 256) return true;
-  const int64_t generic = items_of(p, rows / p.group), tiled = items_of(p, kRows / p.group);
+  if (seq_rows > 32 && seq_rows <= kRows && p.max_seqlen_q <= 64 && span <= 256) return true;
+  const double generic = items_of(p, rows / p.group), tiled = items_of(p, kRows / p.group);
   if (generic <= kCUs && (int64_t)p.num_tokens * p.num_heads < (int64_t)kCUs * rows) return false;
   const bool fresh = p.kv_lens || !p.cu_k || p.cu_k == p.cu_q;
-  const double longest = fresh ? std::min<double>(span, p.max_seqlen_q) : std::max(span - p.page_size + 1, mean);
-  const double average = longest - std::min(mean, longest) / 2;  // over a sequence's items
-  double rounds = (double)generic / kCUs;
+  const double longest = fresh ? std::min<double>(span, p.max_seqlen_q) : std::max(span - .5 * p.page_size, mean);
+  // over a sequence's items
+  const double average = longest <= p.max_seqlen_q ? longest / 2 : longest - std::min(mean, longest) / 2;
+  double rounds = generic / kCUs;
   // mostly cached tokens: items of about one length, so whole rounds
   if (longest > 2 * (p.batch == 1 ? mean : (double)p.max_seqlen_q)) rounds = std::ceil(rounds);
-  const double t_generic = std::max(12 + .044 * longest, rounds * (12 + .044 * average) + (generic > kCUs ? 4 : 0));
-  const double t_tiled = std::max(10 + .057 * longest, (double)tiled / kCUs * (10 + .057 * average));
+  const double t_generic = std::max(12 + .044 * longest, rounds * (12 + .044 * average) + (generic > kCUs ? 5 : 0));
+  const double t_tiled = std::max(10 + .057 * longest, tiled / kCUs * (10 + .057 * average));
   return t_tiled < t_generic;
 }
 
