@@ -93,8 +93,8 @@ int pa_gather_kv(const uint16_t* cache, int32_t num_pages, int32_t page_size,
  * then a work list of (sequence, chunk) pairs.  From 2048 workgroups on,
  * pa_decode orders the pairs by length and deals them over the XCDs (one
  * extra launch); the output does not depend on the order.  Smaller launches
- * of 2 to 256 sequences at head_dim 128 cut their sequences into parts by an
- * even share of the batch's tokens, so the last bits of a sequence's output
+ * of 2 to 256 sequences at head_dim 128 may cut their sequences into parts by
+ * an even share of the batch's tokens, so the last bits of a sequence's output
  * depend on the other lengths.  The workspace is 256-byte aligned.
  */
 size_t pa_decode_workspace_size(int32_t batch, int32_t num_heads, int32_t head_dim,

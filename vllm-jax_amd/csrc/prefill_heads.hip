@@ -5,9 +5,10 @@
 // registers a 32-token step at a time with two barriers a step, the tiles
 // come straight into a four-stage LDS ring and one wave of a SIMD feeds the
 // matrix cores while the other takes its softmax.  16 sequences of 1000 to
-// 3000 tokens, 32 / 8 heads, generic -> this (one MI355X): 64 391 -> 351 us,
-// 96 522 -> 511 (soft cap 852 -> 653), 256 1927 -> 1316 (soft cap 2037 ->
-// 1326); one sequence of 32768 tokens: 64 4.82 -> 4.31 ms, 256 25.1 -> 16.7.
+// 3000 tokens, 32 / 8 heads, generic -> this with the work list (one MI355X):
+// 64 360 -> 316 us (soft cap 481 -> 422), 96 489 -> 440 (828 -> 575), 256 1682
+// -> 1083 (1771 -> 1110); one sequence of 32768 tokens: 64 4.83 -> 4.21 ms, 96
+// 6.55 -> 5.94, 256 24.5 -> 16.6.
 // Bound by the softmax's VALU work at 64, by MFMA and LDS reads at 256, and
 // by the ~7 us an item spends outside its loop at these lengths.  80 gained
 // nothing (492 us against 478, its generic kernel also fits two workgroups a
@@ -83,8 +84,8 @@ static double items_of(const PrefillParams& p, int64_t tokens) {
 // from max_seqlen_q; the others are taken to be as long, or, up to max_seqlen_q,
 // to have nothing cached.
 // Generic -> tiled, 32 / 8 heads unless said, us (both kernels timed at 740
-// shapes, 400 of them with the soft cap as well; this rule is never more than
-// 2 % behind the generic one): generic
+// shapes, 400 of them with the soft cap as well; in all but three this rule is
+// within 2.3 % of the generic one or faster, at worst 1.2 us of 23 behind): generic
 // 3 x 299 tokens 28.0 -> 31.5, 1 x 2000 118 -> 131, 1 x 1000 behind 4000
 // cached 237 -> 302, 16 / 8 heads 1 x 4000 211 -> 246; tiled 4 x 511 50.3 ->
 // 46.6, 1 x 3000 258 -> 190, 4 x 300 behind 4000 384 -> 265, 8 / 8 heads 8 x 64
